@@ -674,7 +674,7 @@ def bench_cfg2(args):
                 frac=tops / FP16_PEAK_TFLOPS, frac_of_int8_peak=tops / INT8_PEAK_TOPS,
                 timing="HIP-graph replay of the MLP block (q3vl_mlp_i8: A's quantizer and "
                        "the two GEMMs)",
-                kernel="quantize_frag_kernel + gemm_mf_kernel: gate|up with the SwiGLU "
+                kernel="quantize_t16_kernel + gemm_t16_kernel: gate|up with the SwiGLU "
                        "epilogue quantizing h into down's operand, then down")
 
 
@@ -736,7 +736,7 @@ def bench_cfg4(args):
                 frac=tops / FP16_PEAK_TFLOPS, frac_of_int8_peak=tops / INT8_PEAK_TOPS,
                 gemms=B * len(VIS_SHAPES) + len(MERGER_SHAPES),
                 timing="HIP-graph replay of the pass (quantizers and GEMMs)",
-                kernel="quantize_frag_kernel + gemm_mf_kernel (K a multiple of 512: every "
+                kernel="quantize_t16_kernel + gemm_t16_kernel (every "
                        "vision and merger linear)")
 
 
@@ -848,7 +848,7 @@ def pmc_workload_gemm():
     2's GEMMs (gate|up with the SwiGLU epilogue, then down, M = 512) and of
     config 4's vision linears (qkv, proj, fc1, fc2 at M = 784; the merger's
     fc1 at M = 196), each call its fragment-order quantizer and its
-    gemm_mf_kernel."""
+    gemm_t16_kernel."""
     import torch
     import q3vl_int8 as q
     shapes = [("cfg2 gate|up", 512, 6144, 2048, True), ("cfg2 down", 512, 2048, 6144, False)]
@@ -1131,7 +1131,7 @@ def main():
     ap.add_argument("--pmc-summary", nargs="+", metavar="DIR",
                     help="print per-dispatch counter averages (and derived GEMM figures) of the "
                          "kernels named by --pmc-match from rocprofv3 --pmc output directories")
-    ap.add_argument("--pmc-match", default="gemm_mf_kernel")
+    ap.add_argument("--pmc-match", default="gemm_t16_kernel")
     ap.add_argument("--pmc-traffic", nargs=2, metavar=("FETCH_DIR", "WRITE_DIR"),
                     help="print the decode GEMVs' HBM traffic summary from the FETCH_SIZE and "
                          "WRITE_SIZE runs of --pmc-workload")

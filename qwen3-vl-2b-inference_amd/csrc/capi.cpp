@@ -208,8 +208,7 @@ int run_linear(const float *A, int nseg, const int8_t *const *W, const float *co
         int cus = 0;
         rc = device_cus(&cus);
         if (rc) return rc;
-        for (int i = 0; wide_mf && i < nseg; ++i)
-            wide_mf = gemm_mf_serves((int)M, (int)Ns[i], (int)K, false, cus);
+        for (int i = 0; wide_mf && i < nseg; ++i) wide_mf = K % 512 == 0;
     }
     if (gemv_path_ok(M, K, gs) && !wide_mf) {
         // Lane numerics apply per segment shape; segments sharing one launch
@@ -259,26 +258,32 @@ int run_linear(const float *A, int nseg, const int8_t *const *W, const float *co
     }
     _Float16 *aq = reinterpret_cast<_Float16 *>(wbase + LG.aq);
     float *asT = reinterpret_cast<float *>(wbase + LG.as);
-    // Group size 64 without group sums: the fragment-order GEMM where it
-    // serves every segment's shape (it addresses its buffers with 32-bit byte
-    // offsets), with the activations quantized into MFMA fragment order; one
-    // GEMM per segment, gate and up together under SwiGLU.
-    bool use_mf = gs == 64 && ((M + 31) & ~(size_t)31) * K * 2 <= 0x7fffffffULL &&
-                  (size_t)Ns[0] * K <= 0x7fffffffULL;
+    // Without group sums: the fragment-order GEMM, one per segment, gate and
+    // up together under SwiGLU.
+    bool use_t16 = true;
+    for (int i = 0; use_t16 && i < nseg; ++i)
+        use_t16 = !(G && G[i]) && gemm_t16_serves((int)M, (int)Ns[i], (int)K, (int)gs);
     int cus = 0;
-    if (use_mf) {
-        rc = device_cus(&cus);
-        if (rc) return rc;
+    rc = device_cus(&cus);
+    if (rc) return rc;
+    if (use_t16 && mode == GEMV_ARGMAX) {
+        // a vocabulary of more partials than the workspace holds: refused at
+        // group size 64, scanned from stored logits at the others
+        const size_t cols = gs == 64 && K % 512 == 0 && M > 32
+                                ? 64 : (size_t)gemm_t16_argmax_cols((int)M, (int)Ns[0], (int)gs, cus);
+        const size_t nparts = (Ns[0] + cols - 1) / cols;
+        if (nparts > kMaxGemvParts) {
+            if (gs == 64 && K % 512 == 0)
+                return fail(Q3VL_ERR_UNSUPPORTED, "argmax: %zu partials exceed %zu", nparts, kMaxGemvParts);
+            use_t16 = false;
+        }
     }
-    for (int i = 0; use_mf && i < nseg; ++i)
-        use_mf = !(G && G[i]) && (size_t)Ns[i] * K <= 0x7fffffffULL &&
-                 gemm_mf_serves((int)M, (int)Ns[i], (int)K, mode == GEMV_SWIGLU, cus);
-    if (use_mf) {
+    if (use_t16) {
         const int Mt = (int)((M + 31) / 32);
         // 5..16 rows against a very wide weight (the lm_head over a batch of
         // rows): 16-row MFMA tiles with the weights loaded straight into the
         // operands, the activations quantized inside the kernel
-        bool wide16 = Mt == 1 && M >= 5 && mode != GEMV_SWIGLU;
+        bool wide16 = Mt == 1 && M >= 5 && gs == 64 && K % 512 == 0 && mode != GEMV_SWIGLU;
         for (int i = 0; wide16 && i < nseg; ++i)
             wide16 = (size_t)Ns[i] * K >= ((size_t)1 << 26) &&
                      gemm_mf_wide_serves((int)M, (int)Ns[i], (int)K);
@@ -302,27 +307,24 @@ int run_linear(const float *A, int nseg, const int8_t *const *W, const float *co
             }
             return Q3VL_OK;
         }
-        Q3VL_HIP(launch_quantize_frag(A, aq, asT, (int)M, (int)K, st), "quantize launch");
+        Q3VL_HIP(launch_quantize_t16(A, aq, asT, (int)M, (int)K, (int)gs, st), "quantize launch");
         if (mode == GEMV_SWIGLU) {
-            GemmMfArgs g{aq, asT, Mt, W[0], S[0], W[1], S[1], C[0], (int)M, (int)Ns[0], (int)K};
-            Q3VL_HIP(launch_gemm_mf(g, true, cus, st), "gemm launch");
+            GemmT16Args g{aq, asT, Mt, W[0], S[0], W[1], S[1], C[0], (int)M, (int)Ns[0], (int)K};
+            Q3VL_HIP(launch_gemm_t16(g, (int)gs, true, cus, st), "gemm launch");
             return Q3VL_OK;
         }
         for (int i = 0; i < nseg; ++i) {
-            GemmMfArgs g{aq, asT, Mt, W[i], S[i], nullptr, nullptr, C[i], (int)M, (int)Ns[i], (int)K};
+            GemmT16Args g{aq, asT, Mt, W[i], S[i], nullptr, nullptr, C[i], (int)M, (int)Ns[i], (int)K};
             int nparts = 0;
             if (mode == GEMV_ARGMAX) {
                 // the GEMM leaves each block's per-row argmax partial; the
                 // logits are stored only when the caller asked for them
                 g.part_val = reinterpret_cast<float *>(wbase + LG.parts_val);
                 g.part_idx = reinterpret_cast<int32_t *>(wbase + LG.parts_idx);
-                const int cols = gemm_mf_argmax_cols((int)M);
+                const int cols = gemm_t16_argmax_cols((int)M, (int)Ns[i], (int)gs, cus);
                 nparts = (int)((Ns[i] + cols - 1) / cols);
-                if ((size_t)nparts > kMaxGemvParts)
-                    return fail(Q3VL_ERR_UNSUPPORTED, "argmax: %d partials exceed %zu", nparts,
-                                kMaxGemvParts);
             }
-            Q3VL_HIP(launch_gemm_mf(g, false, cus, st), "gemm launch");
+            Q3VL_HIP(launch_gemm_t16(g, (int)gs, false, cus, st), "gemm launch");
             if (mode == GEMV_ARGMAX)
                 Q3VL_HIP(launch_argmax_final(g.part_val, g.part_idx, nparts, (int)M, ids, st),
                          "argmax launch");
@@ -643,11 +645,11 @@ static MlpLayout mlp_layout(size_t M, size_t H, size_t I, size_t gs, bool fused)
         L.aq = off;
         off += align256(Mpad * H * 2);
         L.as = off;
-        off += align256(Mpad * (H / 64) * 4);
+        off += align256(Mpad * (H / gs) * 4);
         L.hq = off;
         off += align256(Mpad * I * 2);
         L.hs = off;
-        off += align256(Mpad * (I / 64) * 4);
+        off += align256(Mpad * (I / gs) * 4);
     } else {
         L.h = off;
         off += align256(M * I * 4);
@@ -659,11 +661,16 @@ static MlpLayout mlp_layout(size_t M, size_t H, size_t I, size_t gs, bool fused)
     return L;
 }
 
-static bool mlp_fuses(size_t M, size_t H, size_t I, size_t gs, int cus) {
-    const size_t Mpad = (M + 31) & ~(size_t)31;
-    return M > 8 && gs == 64 && H % 512 == 0 && I % 512 == 0 && Mpad * (H > I ? H : I) * 2 <= 0x7fffffffULL &&
-           H * I <= 0x7fffffffULL && gemm_mf_serves((int)M, (int)I, (int)H, true, cus) &&
-           gemm_mf_serves((int)M, (int)H, (int)I, false, cus);
+// The fused form needs whole chunks of 64 k on both sides. Its scratch stays
+// within what q3vl_mlp_workspace_bytes() reports: at group size 64 with H and
+// I multiples of 512 that covers the fused layout, elsewhere only shapes whose
+// fused layout fits the other form's fuse.
+static bool mlp_fuses(size_t M, size_t H, size_t I, size_t gs) {
+    if (M <= 8 || I == 0 || H % 64 != 0 || I % 64 != 0 || !gs_ok_gemm(gs)) return false;
+    if (!gemm_t16_serves((int)M, (int)I, (int)H, (int)gs) || !gemm_t16_serves((int)M, (int)H, (int)I, (int)gs))
+        return false;
+    return (gs == 64 && H % 512 == 0 && I % 512 == 0) ||
+           mlp_layout(M, H, I, gs, true).total <= mlp_layout(M, H, I, gs, false).total;
 }
 
 size_t q3vl_mlp_workspace_bytes(size_t M, size_t H, size_t I, size_t group_size) {
@@ -686,7 +693,7 @@ int q3vl_mlp_i8(const float *A, const int8_t *Wg, const float *Sg, const int8_t 
     int cus = 0;
     rc = device_cus(&cus);
     if (rc) return rc;
-    const bool fused = I > 0 && mlp_fuses(M, H, I, group_size, cus);
+    const bool fused = mlp_fuses(M, H, I, group_size);
     const MlpLayout L = mlp_layout(M, H, I, group_size, fused);
     char *wbase = nullptr;
     rc = resolve_ws(workspace, workspace_bytes, L.total, &wbase);
@@ -697,13 +704,14 @@ int q3vl_mlp_i8(const float *A, const int8_t *Wg, const float *Sg, const int8_t 
         _Float16 *hq = reinterpret_cast<_Float16 *>(wbase + L.hq);
         float *hs = reinterpret_cast<float *>(wbase + L.hs);
         const int Mt = (int)((M + 31) / 32);
-        Q3VL_HIP(launch_quantize_frag(A, aq, as, (int)M, (int)H, st), "quantize launch");
-        GemmMfArgs gu{aq, as, Mt, Wg, Sg, Wu, Su, nullptr, (int)M, (int)I, (int)H};
+        const int gs = (int)group_size;
+        Q3VL_HIP(launch_quantize_t16(A, aq, as, (int)M, (int)H, gs, st), "quantize launch");
+        GemmT16Args gu{aq, as, Mt, Wg, Sg, Wu, Su, nullptr, (int)M, (int)I, (int)H};
         gu.hq = hq;
         gu.hqs = hs;
-        Q3VL_HIP(launch_gemm_mf(gu, true, cus, st), "gate|up gemm launch");
-        GemmMfArgs dn{hq, hs, Mt, Wd, Sd, nullptr, nullptr, Y, (int)M, (int)H, (int)I};
-        Q3VL_HIP(launch_gemm_mf(dn, false, cus, st), "down gemm launch");
+        Q3VL_HIP(launch_gemm_t16(gu, gs, true, cus, st), "gate|up gemm launch");
+        GemmT16Args dn{hq, hs, Mt, Wd, Sd, nullptr, nullptr, Y, (int)M, (int)H, (int)I};
+        Q3VL_HIP(launch_gemm_t16(dn, gs, false, cus, st), "down gemm launch");
         return Q3VL_OK;
     }
     // the two calls, h in the workspace

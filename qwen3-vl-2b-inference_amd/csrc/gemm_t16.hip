@@ -1,0 +1,815 @@
+// gemm_t16.hip -- int8-weight GEMM for M > 8 at group sizes 32, 64 and 128
+// (gfx950), on 16x16x32 fp16 MFMA tiles with the weights taken straight from
+// their loads into the operands.
+//
+// Reference: the general path of linear_int8_fp32s_int32acc_transpose,
+// matmul/src/cpu_f32a_i8f32sb_f32c_avx2.cpp:477-662: for each output and
+// each K-group g in ascending order, G = sum_{k in g} q[m,k] * w[n,k] exactly
+// (int32), then acc = fma(float(G) * a_s[m,g], w_s[n,g], acc) (:613-617,
+// 652; GCC contracts the multiply-add, which the golden vectors pin).
+//
+// Exactness. q (int16, |q| <= 127 sqrt(128)) and w (int8) are exact in fp16,
+// and every partial sum of one group is an integer below 2^24, so the MFMAs
+// over the group's k with a zero initial accumulator yield G exactly. (A
+// group whose scale is not finite holds q of 0 and -32768 only: its sums are
+// multiples of 2^15 and exact as well.)
+//
+// What bounds it (probes on MI355X at 2.4 GHz): a SIMD issues one fp32
+// instruction of a wave every 4 to 5 cycles with two waves on it (5 to 8 with
+// one), a 16x16x32 MFMA holds the vector pipe for about 9, and a wave's MFMAs
+// and VALU work add up rather than overlap. A 16 x 16 output tile costs per
+// group of 64 two MFMAs, 8 VALU operations of the fold (the reference rounds
+// the product and the sum apart) and its share of widening the weights (16
+// operations a 16-column tile, shared by the block's row tiles): about 25 ns
+// a SIMD, and 29 to 36 measured in the loop. So the kernel is bound by VALU
+// issue, and everything else is kept off the issue slots:
+// * weights and activations reach LDS by loads with an LDS destination (no
+//   registers, no LDS stores; 170 instead of 224 VGPRs at 128 x 256), waited
+//   for by count;
+// * a weight load covers whole 128-byte pieces of 8 rows. Read straight into
+//   the MFMA's lane order (16 rows by 64 bytes) each load cost the vector
+//   cache ~94 cycles instead of ~16: 512 x 2048 x 6144 34.4 -> 27.5 us;
+// * the activation scales ride in one register per 64 rows and reach the
+//   accumulator rows by DPP row broadcast inside the multiply;
+// * fragments are read three row tiles ahead, MFMAs issued one tile ahead of
+//   their fold.
+#include <type_traits>
+
+#include "q3vl_device.hpp"
+#include "q3vl_kernels.hpp"
+
+namespace q3vl {
+
+typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
+typedef float float4_t __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
+// ------------------------------------------------------- activation fragments
+// q in fp16, in chunks of 64 k: per 32-row m-tile t and chunk c a 4 KB block
+// [16-row half][MFMA u][lane][8 halves], lane l holding row l % 16 and the k
+// that its weight bytes hold: with c = l / 16, k = 16c + 8u + j at group
+// sizes 64 and 128 (a lane's 16 weight bytes feed both MFMAs of the chunk),
+// k = 32u + 8c + j at 32 (one group an MFMA). The scales come per m-tile and
+// group as 32 floats [r][4 half + i] of row 16 half + 4r + i: what the 16
+// lanes of DPP row r need for the accumulator rows they hold.
+template <int GS>
+Q3VL_INLINE size_t frag_off(int mt, int row32, int Kc, int k) {
+    const int e = k & 63;
+    const int c = GS == 32 ? (e >> 3) & 3 : e >> 4, u = GS == 32 ? e >> 5 : (e >> 3) & 1;
+    return (((((size_t)mt * Kc + (k >> 6)) * 2 + (row32 >> 4)) * 2 + u) * 64 + (row32 & 15) + 16 * c) * 16 +
+           (e & 7) * 2;
+}
+Q3VL_INLINE size_t frag_scale(int mt, int row32, int Kg, int g) {
+    return ((size_t)mt * Kg + g) * 32 + ((row32 >> 2) & 3) * 8 + 4 * (row32 >> 4) + (row32 & 3);
+}
+
+#define Q3VL_QUAD(v, ctrl) \
+    __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), ctrl, 0xF, 0xF, true))
+
+// The reference quantizer (cpu_f32a_i8f32sb_f32c_avx2.cpp:135-177) of one
+// (row, group) by a quad of lanes: lane j holds x[16v + 4j + c] (cv[v].c), so
+// chains 4j + c of the 16 run in the lane over v ascending; V[i] = P[i] +
+// P[i+8] takes lane j + 2, the fixed tree runs in lane 0. The 4-value pieces
+// go out as fp16 through store(v, halves), the scale from lane 0.
+template <int GS, typename Store>
+Q3VL_INLINE float quant_team(const float4 (&cv)[GS / 16], Store store) {
+    float p0 = 0.0f, p1 = 0.0f, p2 = 0.0f, p3 = 0.0f;
+#pragma unroll
+    for (int v = 0; v < GS / 16; ++v) {
+        p0 = fmaf(cv[v].x, cv[v].x, p0);
+        p1 = fmaf(cv[v].y, cv[v].y, p1);
+        p2 = fmaf(cv[v].z, cv[v].z, p2);
+        p3 = fmaf(cv[v].w, cv[v].w, p3);
+    }
+    // lanes 0, 1 take lanes 2, 3 (quad_perm [2,3,2,3]); lane 0 takes lane 1's
+    // V[4..7] ([1,1,1,1]); lane 0's sum to the quad ([0,0,0,0])
+    const float v0 = p0 + Q3VL_QUAD(p0, 0xEE), v1 = p1 + Q3VL_QUAD(p1, 0xEE);
+    const float v2 = p2 + Q3VL_QUAD(p2, 0xEE), v3 = p3 + Q3VL_QUAD(p3, 0xEE);
+    const float w0 = Q3VL_QUAD(v0, 0x55), w1 = Q3VL_QUAD(v1, 0x55);
+    const float w2 = Q3VL_QUAD(v2, 0x55), w3 = Q3VL_QUAD(v3, 0x55);
+    const float sumsq = Q3VL_QUAD(tree8(v0, v1, v2, v3, w0, w1, w2, w3), 0x00);
+    const float s = group_scale(sumsq, 1.0f / (float)GS);
+    const float inv = rcp_rn(s);
+    // q = rne(x / s): for a finite scale |q| < 2^11, and adding and removing
+    // 1.5 * 2^23 rounds to the integer, ties to even (quant_pair_finite's
+    // integer); otherwise the reference's saturating conversion
+    if (__builtin_expect(__builtin_isfinite(s), 1)) {
+        constexpr float kMagic = 12582912.0f;
+#pragma unroll
+        for (int v = 0; v < GS / 16; ++v) {
+            const float r0 = (cv[v].x * inv + kMagic) - kMagic, r1 = (cv[v].y * inv + kMagic) - kMagic;
+            const float r2 = (cv[v].z * inv + kMagic) - kMagic, r3 = (cv[v].w * inv + kMagic) - kMagic;
+            store(v, __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(r0, r1)),
+                  __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(r2, r3)));
+        }
+    } else {
+#pragma unroll
+        for (int v = 0; v < GS / 16; ++v) {
+            const uint32_t q0 = quant_pair(cv[v].x * inv, cv[v].y * inv);
+            const uint32_t q1 = quant_pair(cv[v].z * inv, cv[v].w * inv);
+            store(v,
+                  __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz((float)(int16_t)(q0 & 0xFFFF),
+                                                                          (float)(int16_t)(q0 >> 16))),
+                  __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz((float)(int16_t)(q1 & 0xFFFF),
+                                                                          (float)(int16_t)(q1 >> 16))));
+        }
+    }
+    return s;
+}
+
+// A block of 128 threads takes 8 rows x 4 groups: a 128-byte line of the
+// fragment order holds 16 bytes of 8 consecutive rows, so every line is
+// written whole by one block.
+template <int GS>
+__global__ __launch_bounds__(128) void quantize_t16_kernel(const float *__restrict__ A,
+                                                           unsigned char *__restrict__ qf,
+                                                           float *__restrict__ asf, int M, int K) {
+    const int Kg = K / GS, Kc = K / 64;
+    const int j = threadIdx.x & 3, team = threadIdx.x >> 2;
+    const int g = blockIdx.x * 4 + (team & 3), m = blockIdx.y * 8 + (team >> 2);
+    if (g >= Kg) return;  // whole quads leave together
+    const bool real = m < M;
+    float4 cv[GS / 16];
+    const float *x = A + (size_t)(real ? m : M - 1) * K + (size_t)g * GS + 4 * j;
+#pragma unroll
+    for (int v = 0; v < GS / 16; ++v) {
+        const float4 f = *reinterpret_cast<const float4 *>(x + 16 * v);
+        cv[v] = real ? f : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    }
+    const float s = quant_team<GS>(cv, [&](int v, uint32_t h0, uint32_t h1) {
+        *reinterpret_cast<uint2 *>(qf + frag_off<GS>(m >> 5, m & 31, Kc, g * GS + 16 * v + 4 * j)) =
+            real ? make_uint2(h0, h1) : make_uint2(0u, 0u);
+    });
+    if (j == 0) asf[frag_scale(m >> 5, m & 31, Kg, g)] = real ? s : 0.0f;
+}
+
+hipError_t launch_quantize_t16(const float *A, _Float16 *qf, float *asf, int M, int K, int gs,
+                               hipStream_t st) {
+    if (K % 64 != 0 || M < 1) return hipErrorInvalidValue;
+    const dim3 grid((K / gs + 3) / 4, (M + 31) / 32 * 4);
+    unsigned char *q = reinterpret_cast<unsigned char *>(qf);
+    if (gs == 32) quantize_t16_kernel<32><<<grid, 128, 0, st>>>(A, q, asf, M, K);
+    else if (gs == 64) quantize_t16_kernel<64><<<grid, 128, 0, st>>>(A, q, asf, M, K);
+    else if (gs == 128) quantize_t16_kernel<128><<<grid, 128, 0, st>>>(A, q, asf, M, K);
+    else return hipErrorInvalidValue;
+    return hipGetLastError();
+}
+
+// ---------------------------------------------------------------- the GEMM
+// 4 int8 bytes -> 4 fp16 values in two dwords (bytes 0, 1 -> lo, 2, 3 -> hi),
+// one conversion a byte: v_cvt_f16_i16 reading the byte sign-extended (SDWA
+// source select) and writing one half of the destination, exact for every
+// int8. The two destinations alternate, so no instruction reads the half that
+// the one right before it wrote.
+Q3VL_INLINE void widen4(uint32_t x, uint32_t &lo, uint32_t &hi) {
+    asm("v_cvt_f16_i16_sdwa %0, sext(%2) dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:BYTE_0\n\t"
+        "v_cvt_f16_i16_sdwa %1, sext(%2) dst_sel:WORD_0 dst_unused:UNUSED_PAD src0_sel:BYTE_2\n\t"
+        "v_cvt_f16_i16_sdwa %0, sext(%2) dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:BYTE_1\n\t"
+        "v_cvt_f16_i16_sdwa %1, sext(%2) dst_sel:WORD_1 dst_unused:UNUSED_PRESERVE src0_sel:BYTE_3"
+        : "=&v"(lo), "=&v"(hi)
+        : "v"(x));
+}
+Q3VL_INLINE half8_t widen8(uint32_t x, uint32_t y) {
+    uint32_t a, b, c, d;
+    widen4(x, a, b);
+    widen4(y, c, d);
+    return __builtin_bit_cast(half8_t, (u32x4){a, b, c, d});
+}
+
+// Loads with an LDS destination: lane l's 16 (4) bytes at voff + soff of the
+// resource go to LDS at lds + 16 l (4 l). Written in asm because the compiler
+// would wait for every such load before any later LDS read; dma_wait<N>()
+// waits until at most N of this wave's loads are in flight (they complete in
+// order).
+typedef uint32_t rsrc_t __attribute__((ext_vector_type(4)));
+Q3VL_INLINE rsrc_t make_rsrc(const void *p, uint32_t bytes) {
+    const uint64_t a = (uint64_t)p;
+    return (rsrc_t){(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a),
+                    (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32)),
+                    (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000u};
+}
+Q3VL_INLINE void dma16(rsrc_t r, int voff, int soff, int lds) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                 :: "s"(lds), "v"(voff), "s"(r), "s"(soff) : "memory");
+#endif
+}
+Q3VL_INLINE void dma4(rsrc_t r, int voff, int soff, int lds) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds"
+                 :: "s"(lds), "v"(voff), "s"(r), "s"(soff) : "memory");
+#endif
+}
+template <int N> Q3VL_INLINE void dma_wait() {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N < 63 ? N : 63) : "memory");  // (the counter's field)
+#endif
+}
+
+// The tile shape. GS: group size. A: 16-row tiles of the block (2, 4 or 8:
+// all of its waves share its rows). B: 16-column tiles of a wave (SwiGLU: B/2
+// gate, B/2 up). NW: waves, side by side along the columns. A unit is UC
+// chunks of 64 k: one group of 64 or 128, two of 32. SU: units of a stage of
+// activations (three in LDS). NB: stages of weights (128 bytes of each row)
+// in LDS per wave.
+template <int GS_, int A_, int B_, int NW_, int SU_, int NB_, bool SWIGLU_> struct T16 {
+    static constexpr int GS = GS_, A = A_, B = B_, NW = NW_, SU = SU_, NB = NB_;
+    static constexpr bool SWIGLU = SWIGLU_;
+    static constexpr int NT = 64 * NW;               // threads
+    static constexpr int NJ = SWIGLU ? B / 2 : B;    // output column tiles of a wave
+    static constexpr int COLS = 16 * NW * NJ;        // output columns of the block
+    static constexpr int MT = A / 2;                 // 32-row m-tiles of the block
+    static constexpr int UC = GS == 128 ? 2 : 1;     // chunks of a unit
+    static constexpr int GU = GS == 32 ? 2 : 1;      // groups of a unit
+    static constexpr int UB = 2 / UC;                // units of a weight stage
+    static constexpr int NM = 2 * UC;                // MFMAs of a tile and unit
+    static constexpr int SC = SU * UC, SG = SU * GU; // chunks, groups of an activation stage
+    static constexpr int NG = 4 * GU;                // groups of the loop body (four units)
+    static constexpr int PD = 3;                     // steps that fragments are read ahead
+    static constexpr int CB = (A - 1 + PD) / A;      // units before the next stage that first read it
+    static constexpr int ABUF = MT * SC * 4096;      // bytes of a stage's fragments
+    static constexpr int NA = ABUF / 1024 / NW;      // loads per wave and stage
+    static constexpr int SBYTES = MT * SG * 128;     // bytes of a stage's scales
+    static constexpr int SBUF = (SBYTES + 1023) / 1024 * 1024;
+    static constexpr int WST = NG / 4;               // w_s loads per column tile and body
+    static constexpr int OFF_S = 3 * ABUF, OFF_B = OFF_S + 3 * SBUF;
+    static constexpr int OFF_W = OFF_B + NW * B * NB * 2048, LDS = OFF_W + NW * 2 * B * WST * 256;
+    static_assert(A == 2 || A == 4 || A == 8, "rows");
+    static_assert(!SWIGLU || B % 2 == 0, "gate and up tiles");
+    static_assert(SU >= CB && 4 % SU == 0 && NA * 1024 * NW == ABUF && SBUF <= 1024 * NW, "stages");
+    static_assert(LDS <= 160 * 1024, "LDS");
+    // Loads that a wave issues between the load a wait is for and the wait, in
+    // the loop's steady state: 'a' the activation stage met at unit us, 'b'
+    // the weight stage first read in unit us, 'w' the next body's w_s. (The
+    // loop is entered with nothing in flight, so its first turns wait for no
+    // less.)
+    static constexpr int behind(char what, int us) {
+        int n = 0, at = -1;  // loads issued so far; count right behind the one waited for
+        for (int pass = 0; pass < 2; ++pass) {
+            n = 0;
+            int target_a = -1, target_b = -1, target_w = -1;
+            // the wait's place: body 5, unit us; what it waits for
+            if (what == 'a') target_a = (20 + us) / SU + 1;
+            if (what == 'b') target_b = (20 + us + 1) / UB;
+            if (what == 'w') target_w = 6;
+            for (int u = 0; u < 24; ++u) {
+                const int su = u % SU;
+                if (su == SU - CB) {
+                    if (pass == 1 && what == 'a' && u == 20 + us) return n - at;
+                    n += NA + 1;
+                    if (u / SU + 2 == target_a) at = n;
+                }
+                if (u % 4 == 0) {
+                    n += B * WST;
+                    if (u / 4 + 2 == target_w) at = n;
+                }
+                if ((u + 1) % UB == 0 && pass == 1 && what == 'b' && u == 20 + us) return n - at;
+                if ((u + 1) % UB == UB - 1) {
+                    n += 2 * B;
+                    if ((u + 1) / UB + NB == target_b) at = n;
+                }
+                if (u % 4 == 3 && pass == 1 && what == 'w' && u == 23) return n - at;
+            }
+        }
+        return 0;
+    }
+};
+
+template <typename T, int MINB, bool HQ>
+__global__ __launch_bounds__(64 * T::NW, MINB) void gemm_t16_kernel(
+    const unsigned char *Af, const float *asf, const int8_t *W0, const float *S0, int Mt, int N,
+    int K, int M, const int8_t *W1, GemmT16Args args) {
+    constexpr int GS = T::GS, A = T::A, B = T::B, NW = T::NW, SU = T::SU, NB = T::NB, NT = T::NT, NJ = T::NJ;
+    constexpr int COLS = T::COLS, MT = T::MT, UC = T::UC, GU = T::GU, UB = T::UB, NM = T::NM, SC = T::SC;
+    constexpr int SG = T::SG, NG = T::NG, PD = T::PD, CB = T::CB, ABUF = T::ABUF, SBUF = T::SBUF, WST = T::WST;
+    constexpr int NAS = (A + 3) / 4;  // scale registers of a group (64 rows each)
+    constexpr bool SWIGLU = T::SWIGLU;
+    extern __shared__ __align__(16) unsigned char smem[];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c = lane >> 4, nl = lane & 15;
+    const int Kc = K / 64, Kg = K / GS;
+    // XCD-aware tile order. Workgroups go to the 8 XCDs round-robin (block b
+    // to XCD b % 8), and each XCD has its own L2: XCD x takes the contiguous
+    // tiles [x per, (x+1) per), M-tile fastest, so a few columns of weight
+    // rows meet all activation rows in one L2.
+    const int tiles_m = (Mt + MT - 1) / MT;
+    const int tiles = tiles_m * ((N + COLS - 1) / COLS);
+    const int per = (tiles + 7) / 8;
+    const int t = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
+    if (t >= tiles || (int)(blockIdx.x / 8) >= per) return;  // whole block: before any barrier
+    const int n0 = (t / tiles_m) * COLS, mt0 = (t % tiles_m) * MT;
+
+    // Buffer resources based at the block's own rows; the advance along K
+    // goes in the scalar offset.
+    const int mtn = min(MT, Mt - mt0), rows = N - n0;
+    const rsrc_t rA = make_rsrc(Af + (size_t)mt0 * Kc * 4096, (uint32_t)mtn * Kc * 4096);
+    const rsrc_t rAS = make_rsrc(asf + (size_t)mt0 * Kg * 32, (uint32_t)mtn * Kg * 128);
+    const rsrc_t rW0 = make_rsrc(W0 + (size_t)n0 * K, (uint32_t)rows * K);
+    const rsrc_t rW1 = make_rsrc((SWIGLU ? W1 : W0) + (size_t)n0 * K, (uint32_t)rows * K);
+    const rsrc_t rS0 = make_rsrc(S0 + (size_t)n0 * Kg, (uint32_t)rows * Kg * 4);
+    const rsrc_t rS1 = make_rsrc((SWIGLU ? args.S1 : S0) + (size_t)n0 * Kg, (uint32_t)rows * Kg * 4);
+
+    // ---- activations: the waves copy a stage's fragments and scales linearly
+    // in 1 KB pieces (m-tiles past the product are clamped; the scales' pieces
+    // repeat over the waves, the same bytes to the same place)
+    int aoff[T::NA], asoff;
+#pragma unroll
+    for (int i = 0; i < T::NA; ++i) {
+        const int p = wid + NW * i, mt = p / (SC * 4);
+        aoff[i] = min(mt, mtn - 1) * Kc * 4096 + (p % (SC * 4)) * 1024 + lane * 16;
+    }
+    const int spiece = wid % (SBUF / 1024);
+    {
+        const int o = min(spiece * 1024 + lane * 16, T::SBYTES - 16), mt = o / (SG * 128);
+        asoff = min(mt, mtn - 1) * Kg * 128 + o % (SG * 128);
+    }
+    // ---- weights: a stage takes 128 bytes of each of a tile's 16 rows, 8 rows
+    // a load: 8 consecutive lanes read one row's 128 bytes (16 lanes spread
+    // over 16 rows, the order the MFMA wants, cost six times as much in the
+    // vector cache). LDS slot 8 row + s holds the row's 16-byte piece s ^
+    // ((row / 2) & 7), so that a fragment read meets 16 different bank groups.
+    // w_s: four groups of each row, 4 lanes a row.
+    int woff[B][2], soff[B];
+#pragma unroll
+    for (int j = 0; j < B; ++j) {
+        const int r0 = 16 * (wid * NJ + j % NJ);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int r = 8 * i + (lane >> 3);
+            woff[j][i] = min(r0 + r, rows - 1) * K + 16 * ((lane & 7) ^ ((r >> 1) & 7));
+        }
+        soff[j] = (min(r0 + (lane >> 2), rows - 1) * Kg + (lane & 3)) * 4;
+    }
+    const int bbase = T::OFF_B + wid * B * NB * 2048, wbase = T::OFF_W + wid * 2 * B * WST * 256;
+    auto load_a = [&](int buf, int stage) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < T::NA; ++i) dma16(rA, aoff[i], stage * SC * 4096, buf * ABUF + (wid + NW * i) * 1024);
+        dma16(rAS, asoff, stage * SG * 128, T::OFF_S + buf * SBUF + spiece * 1024);
+    };
+    auto load_b = [&](int sl, int stage) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < B; ++j)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                dma16(SWIGLU && j >= NJ ? rW1 : rW0, woff[j][i], stage * 128, bbase + (j * NB + sl) * 2048 + i * 1024);
+    };
+    auto load_ws = [&](int sl, int body) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < B; ++j)
+#pragma unroll
+            for (int h = 0; h < WST; ++h)
+                dma4(SWIGLU && j >= NJ ? rS1 : rS0, soff[j], (body * NG + 4 * h) * 4, wbase + ((sl * B + j) * WST + h) * 256);
+    };
+
+    float4_t out[A][B];
+#pragma unroll
+    for (int i = 0; i < A; ++i)
+#pragma unroll
+        for (int j = 0; j < B; ++j) out[i][j] = (float4_t){0.0f, 0.0f, 0.0f, 0.0f};
+
+    // this lane's place in a group's scales of a 64-row range: DPP row r's 16
+    // lanes hold what rows 16 i + 4r + e need, in lane 4 i + e
+    const int asl = (A >= 4 ? ((lane >> 3) & 1) * SG * 32 : 0) + (lane >> 4) * 8 + (lane & 7);
+    const float4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    half8_t fr[4][NM];                 // activation fragments of four steps
+    float4_t acc[2][B][GU];            // group sums of two steps
+    u32x4 raw[B][UC];                  // the next unit's weights
+    uint32_t bf[2][B][NM][4];          // widened weights of two units
+    float as[2][GU][NAS];              // scales of two units
+    float wsn[B][NG];                  // the next body's w_s
+    // fragments of row tile i / the scales of unit u of the stage in buffer buf
+    auto read_fr = [&](int sl, int buf, int u, int i) __attribute__((always_inline)) {
+        const u32x4 *p = reinterpret_cast<const u32x4 *>(smem + buf * ABUF) + ((i >> 1) * SC + u * UC) * 256 + (i & 1) * 128 + lane;
+#pragma unroll
+        for (int k = 0; k < NM; ++k) fr[sl][k] = __builtin_bit_cast(half8_t, p[(k >> 1) * 256 + (k & 1) * 64]);
+    };
+    auto read_as = [&](int sl, int buf, int u) __attribute__((always_inline)) {
+        const float *p = reinterpret_cast<const float *>(smem + T::OFF_S + buf * SBUF);
+#pragma unroll
+        for (int g = 0; g < GU; ++g)
+#pragma unroll
+            for (int n = 0; n < NAS; ++n) as[sl][g][n] = p[n * 2 * SG * 32 + (u * GU + g) * 32 + asl];
+    };
+    // this lane's weights of unit u of the stage in slot sl
+    auto read_raw = [&](int sl, int u) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < B; ++j) {
+            const unsigned char *p = smem + bbase + (j * NB + sl) * 2048 + nl * 128;
+#pragma unroll
+            for (int x = 0; x < UC; ++x) {
+                if constexpr (GS == 32) {  // 8 bytes of each of the chunk's two groups
+                    const u32x2 g0 = *reinterpret_cast<const u32x2 *>(p + (((4 * u + (c >> 1)) ^ (nl >> 1)) & 7) * 16 + 8 * (c & 1));
+                    const u32x2 g1 = *reinterpret_cast<const u32x2 *>(p + (((4 * u + 2 + (c >> 1)) ^ (nl >> 1)) & 7) * 16 + 8 * (c & 1));
+                    raw[j][x] = (u32x4){g0[0], g0[1], g1[0], g1[1]};
+                } else {
+                    raw[j][x] = *reinterpret_cast<const u32x4 *>(p + (((4 * (u * UC + x) + c) ^ (nl >> 1)) & 7) * 16);
+                }
+            }
+        }
+    };
+    auto read_ws = [&](int sl) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < B; ++j)
+#pragma unroll
+            for (int h = 0; h < WST; ++h) {
+                const float4 v = *reinterpret_cast<const float4 *>(smem + wbase + ((sl * B + j) * WST + h) * 256 + nl * 16);
+                wsn[j][4 * h] = v.x;
+                wsn[j][4 * h + 1] = v.y;
+                wsn[j][4 * h + 2] = v.z;
+                wsn[j][4 * h + 3] = v.w;
+            }
+    };
+    // MFMA k of a step's tiles
+    auto mfma = [&](int fs, int sl, int bs, int k) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < B; ++j) {
+            const half8_t b = __builtin_bit_cast(half8_t, (u32x4){bf[bs][j][k][0], bf[bs][j][k][1], bf[bs][j][k][2], bf[bs][j][k][3]});
+            const int g = GU == 2 ? k : 0;
+            acc[sl][j][g] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fr[fs][k], b, (GU == 2 || k == 0) ? zero : acc[sl][j][g], 0, 0, 0);
+        }
+    };
+    // out = fma(G * a_s, w_s, out) (reference order): the product first, a_s
+    // coming by DPP row broadcast, the sum in a second pass over the same
+    // elements (each product has its own register: one reused right away
+    // would wait out a hazard)
+    auto scale1 = [&](float a_s, float g, int ctrl) __attribute__((always_inline)) {
+        const int v = __builtin_bit_cast(int, a_s);
+        int b = 0;
+        switch (ctrl) {  // (an immediate operand)
+#define Q3VL_C(X) case X: b = __builtin_amdgcn_mov_dpp(v, 0x150 + X, 0xF, 0xF, true); break;
+            Q3VL_C(0) Q3VL_C(1) Q3VL_C(2) Q3VL_C(3) Q3VL_C(4) Q3VL_C(5) Q3VL_C(6) Q3VL_C(7)
+            Q3VL_C(8) Q3VL_C(9) Q3VL_C(10) Q3VL_C(11) Q3VL_C(12) Q3VL_C(13) Q3VL_C(14) Q3VL_C(15)
+#undef Q3VL_C
+        }
+        return __builtin_bit_cast(float, b) * g;
+    };
+    // part k of NM of the folds of step i (us: the unit's place in the body;
+    // sums in acc[sl]): elements x of group g, tile x / 4
+    constexpr int FE = GU == 2 ? 4 * B : 4 * B / NM;
+    auto scale = [&](int i, int us, int sl, int k, float (&tt)[FE]) __attribute__((always_inline)) {
+        const int g = GU == 2 ? k : 0, x0 = GU == 2 ? 0 : k * FE;
+#pragma unroll
+        for (int y = 0; y < FE; ++y)
+            tt[y] = scale1(as[us & 1][g][i / 4], acc[sl][(x0 + y) / 4][g][(x0 + y) % 4], 4 * (i % 4) + (x0 + y) % 4);
+    };
+    auto fold = [&](int i, int us, int k, const float (&tt)[FE], const float (&ws)[B][NG]) __attribute__((always_inline)) {
+        const int g = GU == 2 ? k : 0, x0 = GU == 2 ? 0 : k * FE;
+#pragma unroll
+        for (int y = 0; y < FE; ++y)
+            out[i][(x0 + y) / 4][(x0 + y) % 4] = fmaf(tt[y], ws[(x0 + y) / 4][us * GU + g], out[i][(x0 + y) / 4][(x0 + y) % 4]);
+    };
+    // dword d of B * UC * 4 of raw, widened into bf[bs]
+    auto widen = [&](int bs, int d) __attribute__((always_inline)) {
+        const int j = d / (UC * 4), u = d / 4 % UC, w = d % 4;
+        widen4(raw[j][u][w], bf[bs][j][2 * u + w / 2][2 * (w & 1)], bf[bs][j][2 * u + w / 2][2 * (w & 1) + 1]);
+    };
+    constexpr int ND = B * UC * 4;           // dwords to widen per unit
+    constexpr int NSUB = (A - 1) * NM;       // sub-steps that widen (the next unit's first MFMA follows)
+
+    const int nbody = Kc / (4 * UC), last = 4 * nbody - 1, lasta = last / SU, lastb = last / UB;
+    int b0 = 0, b1 = 1, b2 = 2;  // activation buffers of this, the next and the stage after
+    int sb = 0;                  // weight slot of the stage that holds the next unit
+    // One unit n (us: its place among the four of the loop body). On entry its
+    // weights are widened in bf[us & 1], its scales read, the fragments of
+    // steps 0 .. PD-1 read and step 0's MFMAs issued.
+    auto unit = [&](auto usc, int n, const float (&ws)[B][NG]) __attribute__((always_inline)) {
+        constexpr int us = decltype(usc)::value, su = us % SU;
+        if constexpr (su == SU - CB) {
+            // the next stage has landed for every wave, and every wave is past
+            // the previous one, whose buffer the stage after the next takes
+            dma_wait<T::behind('a', us)>();
+            lds_barrier();
+            load_a(b2, min(n / SU + 2, lasta));
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (us == 0) load_ws((n >> 2) & 1, min((n >> 2) + 2, nbody - 1));
+        if constexpr ((us + 1) % UB == 0) dma_wait<T::behind('b', us)>();
+        read_raw(sb, (us + 1) % UB);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < A; ++i) {
+            // fragments PD steps ahead, MFMAs one step ahead, folds of this one
+            const int st = us * A + i, ru = su + (i + PD) / A;
+            if (i == A - 1) read_as((us + 1) & 1, su == SU - 1 ? b1 : b0, (su + 1) % SU);
+            read_fr((st + PD) & 3, ru >= SU ? (ru >= 2 * SU ? b2 : b1) : b0, ru % SU, (i + PD) % A);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int k = 0; k < NM; ++k) {
+                float tt[FE];
+                mfma((st + 1) & 3, (i + 1) & 1, i + 1 < A ? us & 1 : (us + 1) & 1, k);
+                __builtin_amdgcn_sched_barrier(0);
+                scale(i, us, i & 1, k, tt);
+                __builtin_amdgcn_sched_barrier(0);
+                if (i + 1 < A) {
+                    const int sub = i * NM + k;
+#pragma unroll
+                    for (int x = 0; x < ND; ++x)
+                        if (x * NSUB / ND == sub) widen((us + 1) & 1, x);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                fold(i, us, k, tt, ws);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (i + 2 == A && (us + 1) % UB == UB - 1) {  // the slot is consumed
+                load_b(sb, min((n + 1) / UB + NB, lastb));
+                sb = sb + 1 == NB ? 0 : sb + 1;
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        if constexpr (us == 3) {
+            dma_wait<T::behind('w', 3)>();
+            read_ws(((n >> 2) + 1) & 1);
+        }
+        if constexpr (su == SU - 1) {
+            const int x = b0;
+            b0 = b1;
+            b1 = b2;
+            b2 = x;
+        }
+    };
+    static_assert(2 * SU > SU - 1 + (A - 1 + PD) / A, "fragments are read at most one stage ahead");
+
+    if (nbody > 0) {
+        load_a(0, 0);
+        load_a(1, min(1, lasta));
+#pragma unroll
+        for (int x = 0; x < NB; ++x) load_b(x, min(x, lastb));
+        load_ws(0, 0);
+        load_ws(1, min(1, nbody - 1));
+        dma_wait<0>();
+        lds_barrier();
+        read_ws(0);
+        read_as(0, 0, 0);
+#pragma unroll
+        for (int x = 0; x < PD; ++x) read_fr(x, x / A >= SU ? 1 : 0, x / A % SU, x % A);
+        read_raw(0, 0);
+#pragma unroll
+        for (int x = 0; x < ND; ++x) widen(0, x);
+        if (UB == 1) {
+            __builtin_amdgcn_sched_barrier(0);
+            load_b(0, min(NB, lastb));
+            sb = 1;
+        }
+#pragma unroll
+        for (int k = 0; k < NM; ++k) mfma(0, 0, 0, k);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    for (int q = 0; q < nbody; ++q) {
+        float ws[B][NG];
+#pragma unroll
+        for (int j = 0; j < B; ++j)
+#pragma unroll
+            for (int k = 0; k < NG; ++k) ws[j][k] = wsn[j][k];
+        unit(std::integral_constant<int, 0>{}, 4 * q, ws);
+        unit(std::integral_constant<int, 1>{}, 4 * q + 1, ws);
+        unit(std::integral_constant<int, 2>{}, 4 * q + 2, ws);
+        unit(std::integral_constant<int, 3>{}, 4 * q + 3, ws);
+    }
+    dma_wait<0>();  // (the loads past the last unit)
+    // units past the whole bodies (K not a multiple of 256 UC): one at a time
+    const int u0 = 4 * nbody, nu = Kc / UC;
+    for (int n = u0; n < nu; ++n) {
+        lds_barrier();  // the buffer is free
+        for (int p = tid; p < MT * UC * 256; p += NT) {
+            const int mt = p / (UC * 256), r = p % (UC * 256);
+            *reinterpret_cast<u32x4 *>(smem + (mt * SC * 256 + r) * 16) = *reinterpret_cast<const u32x4 *>(
+                Af + ((size_t)(mt0 + min(mt, mtn - 1)) * Kc + n * UC) * 4096 + r * 16);
+        }
+        for (int p = tid; p < MT * GU * 32; p += NT) {
+            const int mt = p / (GU * 32), r = p % (GU * 32);
+            reinterpret_cast<float *>(smem + T::OFF_S)[mt * SG * 32 + r] =
+                asf[((size_t)(mt0 + min(mt, mtn - 1)) * Kg + n * GU) * 32 + r];
+        }
+        float ws[B][NG];
+#pragma unroll
+        for (int j = 0; j < B; ++j) {
+            const int row = n0 + min(16 * (wid * NJ + j % NJ) + nl, rows - 1);
+            const int8_t *w = (SWIGLU && j >= NJ ? W1 : W0) + (size_t)row * K + (size_t)n * UC * 64;
+            const float *s = (SWIGLU && j >= NJ ? args.S1 : S0) + (size_t)row * Kg + n * GU;
+#pragma unroll
+            for (int k = 0; k < GU; ++k) ws[j][k] = s[k];
+#pragma unroll
+            for (int x = 0; x < UC; ++x) {
+                if constexpr (GS == 32) {
+                    const u32x2 g0 = *reinterpret_cast<const u32x2 *>(w + 8 * c), g1 = *reinterpret_cast<const u32x2 *>(w + 32 + 8 * c);
+                    raw[j][x] = (u32x4){g0[0], g0[1], g1[0], g1[1]};
+                } else {
+                    raw[j][x] = *reinterpret_cast<const u32x4 *>(w + 64 * x + 16 * c);
+                }
+            }
+        }
+        lds_barrier();
+        read_as(0, 0, 0);
+#pragma unroll
+        for (int x = 0; x < ND; ++x) widen(0, x);
+#pragma unroll
+        for (int i = 0; i < A; ++i) {
+            read_fr(0, 0, 0, i);
+#pragma unroll
+            for (int k = 0; k < NM; ++k) mfma(0, 0, 0, k);
+#pragma unroll
+            for (int k = 0; k < NM; ++k) {
+                float tt[FE];
+                scale(i, 0, 0, k, tt);
+                fold(i, 0, k, tt, ws);
+            }
+        }
+    }
+    lds_barrier();
+
+    // ---- SwiGLU with hq: the block's h tile (16 A rows x COLS columns, whole
+    // groups of the down projection's K) quantized straight into the down
+    // GEMM's operand in place of storing h. Rows past M get q = 0 and a_s = 0,
+    // as the quantizer's padding rows do.
+    if constexpr (SWIGLU && HQ) {
+        constexpr int HLD = COLS + 4;
+        static_assert(COLS % GS == 0, "whole groups");
+        float *ht = reinterpret_cast<float *>(smem);  // (the last barrier has passed)
+#pragma unroll
+        for (int i = 0; i < A; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    ht[(16 * i + 4 * c + e) * HLD + 16 * (wid * NJ + j) + nl] =
+                        silu_mul(out[i][j][e], out[i][j + NJ][e]);
+        lds_barrier();
+        constexpr int GB = COLS / GS;  // groups of the tile
+        for (int p = tid; p < 16 * A * GB * 4; p += NT) {
+            const int j = p & 3, g = (p >> 2) % GB, rr = (p >> 2) / GB;
+            const int mt = mt0 + (rr >> 5), r = rr & 31;
+            const bool real = 32 * mt + r < M;
+            float4 cv[GS / 16];
+#pragma unroll
+            for (int v = 0; v < GS / 16; ++v)
+                cv[v] = real ? *reinterpret_cast<const float4 *>(ht + rr * HLD + g * GS + 16 * v + 4 * j)
+                             : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            const bool in = mt < Mt && n0 + g * GS < N;  // (a block's last tiles may lie past the product)
+            const float s = quant_team<GS>(cv, [&](int v, uint32_t h0, uint32_t h1) {
+                if (in)
+                    *reinterpret_cast<uint2 *>(reinterpret_cast<unsigned char *>(args.hq) +
+                                               frag_off<GS>(mt, r, N / 64, n0 + g * GS + 16 * v + 4 * j)) =
+                        real ? make_uint2(h0, h1) : make_uint2(0u, 0u);
+            });
+            if (in && j == 0) args.hqs[frag_scale(mt, r, N / GS, n0 / GS + g)] = real ? s : 0.0f;
+        }
+        return;
+    }
+
+    // ---- greedy-argmax partials of the block's columns (plain products): per
+    // row the larger value, equal values the lower column, values that are
+    // not above -FLT_MAX never win -- the strict > scan from -FLT_MAX. Each
+    // lane reduces its B columns, the 16 lanes of a row group by xor shuffles,
+    // the waves through LDS (free: the last barrier has passed).
+    if constexpr (!SWIGLU) {
+        if (args.part_val) {  // uniform
+            float *rv = reinterpret_cast<float *>(smem);  // [NW][16 A]
+            int32_t *ri = reinterpret_cast<int32_t *>(rv + NW * 16 * A);
+#pragma unroll
+            for (int i = 0; i < A; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    float bv = -FLT_MAX;
+                    int32_t bi = -1;
+#pragma unroll
+                    for (int j = 0; j < B; ++j) {
+                        const int col = n0 + 16 * (wid * B + j) + nl;
+                        if (col < N && out[i][j][e] > -FLT_MAX) am_combine(bv, bi, out[i][j][e], col);
+                    }
+#pragma unroll
+                    for (int off = 8; off > 0; off >>= 1) {
+                        const float ov = __shfl_xor(bv, off);
+                        const int32_t oi = __shfl_xor(bi, off);
+                        am_combine(bv, bi, ov, oi);
+                    }
+                    if (nl == 0) {
+                        rv[wid * 16 * A + 16 * i + 4 * c + e] = bv;
+                        ri[wid * 16 * A + 16 * i + 4 * c + e] = bi;
+                    }
+                }
+            lds_barrier();
+            for (int r = tid; r < 16 * A; r += NT) {
+                float bv = -FLT_MAX;
+                int32_t bi = -1;
+#pragma unroll
+                for (int w = 0; w < NW; ++w) am_combine(bv, bi, rv[w * 16 * A + r], ri[w * 16 * A + r]);
+                const int mrow = 32 * mt0 + r;
+                if (mrow < M) {
+                    args.part_val[(size_t)(n0 / COLS) * M + mrow] = bv;
+                    args.part_idx[(size_t)(n0 / COLS) * M + mrow] = bi;
+                }
+            }
+        }
+    }
+
+    // ---- store (an argmax caller that wants no logits passes C = null)
+    if (!args.C) return;  // uniform
+#pragma unroll
+    for (int i = 0; i < A; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int mrow = 32 * mt0 + 16 * i + 4 * c + e;
+            if (mrow >= M) continue;
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                const int col = n0 + 16 * (wid * NJ + j) + nl;
+                if (col < N)
+                    args.C[(size_t)mrow * N + col] = SWIGLU ? silu_mul(out[i][j][e], out[i][SWIGLU ? j + NJ : j][e])
+                                                            : out[i][j][e];
+            }
+        }
+}
+
+template <typename T, int MINB, bool HQ = false>
+static hipError_t launch_t16(const GemmT16Args &a, hipStream_t st) {
+    const int tiles = ((a.N + T::COLS - 1) / T::COLS) * ((a.Mt + T::MT - 1) / T::MT);
+    const int grid = 8 * ((tiles + 7) / 8);
+    constexpr int htile = HQ ? 16 * T::A * (T::COLS + 4) * 4 : 0;
+    constexpr int am = T::SWIGLU ? 0 : T::NW * 16 * T::A * 8;
+    constexpr int lds = T::LDS > htile ? (T::LDS > am ? T::LDS : am) : htile;
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_t16_kernel<T, MINB, HQ>),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (attr != hipSuccess) return attr;
+    gemm_t16_kernel<T, MINB, HQ><<<grid, 64 * T::NW, lds, st>>>(reinterpret_cast<const unsigned char *>(a.Af), a.asf, a.W0,
+                                                               a.S0, a.Mt, a.N, a.K, a.M, a.W1, a);
+    return hipGetLastError();
+}
+
+// Which tile, from timings on MI355X (us a GEMM, weights rotating through
+// more than the L2s; a unit is one group of 64). The fixed cost of a unit in
+// a block falls with the tile (a 32 x 128 block takes 0.29 us a unit, 64 x 128
+// 0.45, or 0.73 for two blocks on a CU, 128 x 128 0.65), so a product too
+// small to give every CU a block runs the fewest rows a block, and a large
+// one the tile whose rounds over the device cost least:
+// * 32 x 64 while its blocks fit the CUs: 64 x 2048 x 2048 8.4 (32 x 128:
+//   9.8; the 32 x 32-tile GEMM before it 14.5);
+// * 32 x 128 while its blocks fit: 512 x 2048 x 6144 27.5 (64 x 128: 44; 42
+//   before), 784 x 1024 x 4096 18.9 (31; 32 before);
+// * then 64 x 128 or 128 x 128: 1000 x 2048 x 6144 48 (128 x 128: 63), 1501 x
+//   2048 x 6144 65 (64 x 128: 70; 92 before).
+// SwiGLU (output columns; each has a gate and an up column): 32 x 64 up to two
+// blocks a CU (64 x 6144 x 2048: 14.5, 64 x 64: 21), 64 x 128 while its blocks
+// fit the CUs (300 rows: 31, 128 x 128: 44; 43 before), else 128 x 128 (1501
+// rows: 132, 64 x 128: 136; 149 before). At group 128 the tiles hold 128
+// columns (whole groups of the h they quantize) and at most 64 rows (more
+// spill).
+static int t16_tile(int M, int N, int gs, bool swiglu, int cus) {
+    auto blocks = [&](int r, int c) { return (long)((M + r - 1) / r) * ((N + c - 1) / c); };
+    if (swiglu) {
+        if (gs == 128) return blocks(32, 128) <= cus ? 0 : 1;
+        if (blocks(32, 64) <= 2L * cus) return 0;
+        return blocks(64, 128) <= cus ? 1 : 2;
+    }
+    if (blocks(32, 64) <= cus) return 0;
+    if (blocks(32, 128) <= cus) return 1;
+    const long b2 = blocks(64, 128);
+    const long c2 = b2 <= cus ? 45 : (b2 + 2 * cus - 1) / (2 * cus) * 73;
+    const long c3 = (blocks(128, 128) + cus - 1) / cus * 65;
+    return c2 <= c3 ? 2 : 3;
+}
+
+// Columns per argmax partial of a plain product.
+int gemm_t16_argmax_cols(int M, int N, int gs, int cus) {
+    return t16_tile(M, N, gs, false, cus) == 0 ? 64 : 128;
+}
+
+// The kernel addresses a block's rows with 32-bit byte offsets.
+bool gemm_t16_serves(int M, int N, int K, int gs) {
+    return (gs == 32 || gs == 64 || gs == 128) && K > 0 && K % 64 == 0 && K % gs == 0 && K <= (1 << 22) && M >= 1 &&
+           N >= 1;
+}
+
+template <int GS> static hipError_t launch_gs(const GemmT16Args &a, bool swiglu, int cus, hipStream_t st) {
+    const int tile = t16_tile(a.M, a.N, GS, swiglu, cus);
+    constexpr int S4 = GS == 128 ? 2 : 4;  // a stage of 256 k (the loads of more do not fit the counter)
+    if (swiglu) {
+        constexpr int NW = GS == 128 ? 8 : 4;
+        using T0 = T16<GS, 2, 2, NW, 2, 2, true>;
+        using T1 = T16<GS, 4, 2, 8, 1, 2, true>;
+        using T2 = T16<GS, GS == 128 ? 4 : 8, 2, 8, 1, 2, true>;
+        if (a.hq)
+            return tile == 0 ? launch_t16<T0, 8 / NW, true>(a, st)
+                             : tile == 1 ? launch_t16<T1, 1, true>(a, st) : launch_t16<T2, 1, true>(a, st);
+        return tile == 0 ? launch_t16<T0, 8 / NW>(a, st)
+                         : tile == 1 ? launch_t16<T1, 1>(a, st) : launch_t16<T2, 1>(a, st);
+    }
+    if (tile == 0) return launch_t16<T16<GS, 2, 1, 4, S4, 3, false>, 1>(a, st);
+    if (tile == 1) return launch_t16<T16<GS, 2, 1, 8, S4, 2, false>, 1>(a, st);
+    if (tile == 2) return launch_t16<T16<GS, 4, 1, 8, 1, 2, false>, 2>(a, st);
+    return launch_t16<T16<GS, 8, 1, 8, 1, 2, false>, 1>(a, st);
+}
+
+hipError_t launch_gemm_t16(const GemmT16Args &a, int gs, bool swiglu, int cus, hipStream_t st) {
+    if (!gemm_t16_serves(a.M, a.N, a.K, gs) || a.Mt != (a.M + 31) / 32) return hipErrorInvalidValue;
+    if (swiglu && a.part_val) return hipErrorInvalidValue;
+    // h quantized in the epilogue: SwiGLU only, whole groups and chunks
+    if (a.hq && (!swiglu || !a.hqs || a.N % 64 != 0 || a.N % gs != 0)) return hipErrorInvalidValue;
+    if (gs == 32) return launch_gs<32>(a, swiglu, cus, st);
+    if (gs == 64) return launch_gs<64>(a, swiglu, cus, st);
+    return launch_gs<128>(a, swiglu, cus, st);
+}
+
+}  // namespace q3vl

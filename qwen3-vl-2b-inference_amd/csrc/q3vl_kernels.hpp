@@ -118,39 +118,39 @@ struct GemmArgs {
 };
 hipError_t launch_gemm(const GemmArgs &a, hipStream_t st);
 
-// Group size 64: activations quantized into MFMA fragment order
-// (launch_quantize_frag), then the fragment-order GEMM.
-struct GemmMfArgs {
-    const _Float16 *Af;  // [Mt][K/64][4][64][8] fp16 fragments of q (Mt = ceil(M/32))
-    const float *asf;    // [Mt][K/64][2][16] activation scales in accumulator order
+// Activations quantized into 16-row MFMA fragments (launch_quantize_t16) and
+// the GEMM over them (group size 32, 64 or 128).
+struct GemmT16Args {
+    const _Float16 *Af;  // [Mt][K/64][2][2][64][8] fp16 fragments of q (Mt = ceil(M/32))
+    const float *asf;    // [Mt][K/gs][32] activation scales in accumulator order
     int Mt;
     const int8_t *W0;    // [N, K] (gate when swiglu)
-    const float *S0;     // [N, K/64]
+    const float *S0;     // [N, K/gs]
     const int8_t *W1;    // up weights when swiglu, else null
     const float *S1;
     float *C;            // [M, N] (H when swiglu)
     int M, N, K;
     // optional (not with swiglu): greedy-argmax partials of each block's
-    // columns per row, [ceil(N / gemm_mf_argmax_cols(...))][M], for
+    // columns per row, [ceil(N / gemm_t16_argmax_cols(...))][M], for
     // launch_argmax_final
     float *part_val = nullptr;
     int32_t *part_idx = nullptr;
-    // optional (swiglu, N % 64 == 0): H is not stored; instead it is
-    // quantized as launch_quantize_frag would quantize it, into hq
-    // [Mt][N/64][4][64][8] and hqs [Mt][N/64][2][16] (the operand of a GEMM
-    // with K = N)
+    // optional (swiglu, N a multiple of 64 and of the group size): H is not
+    // stored but quantized, as launch_quantize_t16 would quantize it, into
+    // the fragments hq and scales hqs of a GEMM with K = N
     _Float16 *hq = nullptr;
     float *hqs = nullptr;
 };
-// Columns per argmax partial of launch_gemm_mf for an M-row plain product.
-int gemm_mf_argmax_cols(int M);
-// qf must hold 32*ceil(M/32)*K halves, asf 32*ceil(M/32)*K/64 floats.
-hipError_t launch_quantize_frag(const float *A, _Float16 *qf, float *asf, int M, int K,
-                                hipStream_t st);
-// Whether the fragment-order GEMM serves an M x N x K product (else
-// launch_gemm's kernels, with launch_quantize_f16), on a device of `cus` CUs.
-bool gemm_mf_serves(int M, int N, int K, bool swiglu, int cus);
-hipError_t launch_gemm_mf(const GemmMfArgs &a, bool swiglu, int cus, hipStream_t st);
+// qf must hold 32*ceil(M/32)*K halves, asf 32*ceil(M/32)*K/gs floats.
+hipError_t launch_quantize_t16(const float *A, _Float16 *qf, float *asf, int M, int K, int gs,
+                               hipStream_t st);
+// Whether this GEMM serves an M x N x K product (else launch_gemm's kernel,
+// with launch_quantize_f16).
+bool gemm_t16_serves(int M, int N, int K, int gs);
+// Columns per argmax partial of a plain product.
+int gemm_t16_argmax_cols(int M, int N, int gs, int cus);
+hipError_t launch_gemm_t16(const GemmT16Args &a, int gs, bool swiglu, int cus, hipStream_t st);
+
 // 16 or fewer rows of fp32 activations A [M, K] against a wide weight (K %
 // 512 == 0, K <= 2048): quantized inside the kernel, 16 x 16 MFMA tiles with
 // the weights loaded straight into the operands. With argmax partial buffers

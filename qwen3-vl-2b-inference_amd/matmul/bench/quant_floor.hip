@@ -106,14 +106,14 @@ int main() {
         CHECK(hipMalloc(&cq, na * 2));
         const size_t n4 = na / 4;
         const unsigned cgrid = (unsigned)((n4 + 255) / 256);
-        auto quant = [&](int r) { return q3vl::launch_quantize_frag(A[r % NA], qf, as, M, K, st); };
+        auto quant = [&](int r) { return q3vl::launch_quantize_t16(A[r % NA], qf, as, M, K, 64, st); };
         auto copy = [&](int r) {
             copy_half_kernel<<<cgrid, 256, 0, st>>>(reinterpret_cast<const float4 *>(A[r % NA]), cq, n4);
             return hipGetLastError();
         };
         auto gemm = [&](int r) {
-            q3vl::GemmMfArgs g{qf, as, Mt, W[r % NW], S[r % NW], nullptr, nullptr, C, M, N, K};
-            return q3vl::launch_gemm_mf(g, false, cus, st);
+            q3vl::GemmT16Args g{qf, as, Mt, W[r % NW], S[r % NW], nullptr, nullptr, C, M, N, K};
+            return q3vl::launch_gemm_t16(g, 64, false, cus, st);
         };
         float q_hot, q_cold, c_hot, c_cold, g_alone, pair;
         if (time_graph(st, reps, [&](int) { return quant(0); }, &q_hot)) return 1;

@@ -1,0 +1,84 @@
+"""GPU parity of the fragment-order GEMM (csrc/gemm_t16.hip): every tile that
+its size rule picks, at each group size, with ragged rows and columns and with
+K of whole loop bodies, of less than one, and of one and a remainder. Against
+the CPU oracle, bit for bit (integer sums are exact and the fp32 order is
+fixed, so there is no tolerance to derive)."""
+import numpy as np
+import pytest
+
+from golden.gen import make_case
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+import q3vl_int8 as q  # noqa: E402
+
+
+def dev(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def assert_bits(got, want, what):
+    torch.cuda.synchronize()
+    g, w = got.cpu().numpy().view(np.uint32), np.ascontiguousarray(want, np.float32).view(np.uint32)
+    bad = np.flatnonzero(g.ravel() != w.ravel())
+    assert bad.size == 0, f"{what}: {bad.size} of {g.size} differ, first at {bad[:5]}"
+
+
+# rows x columns that reach the four plain tiles on 256 CUs (32 x 64, 32 x
+# 128, 64 x 128, 128 x 128), each with ragged last tiles
+PLAIN = [(9, 70), (33, 130), (70, 6001), (70, 14003), (70, 20005), (131, 12801)]
+
+
+@pytest.mark.parametrize("gs", [32, 64, 128])
+@pytest.mark.parametrize("M,N", PLAIN, ids=str)
+def test_linear_tiles(orc, M, N, gs):
+    for K in ((128, 640, 1152) if gs == 128 else (64, 320, 576)):
+        if N > 10000 and K > 700:
+            continue  # (the oracle's time)
+        A, W, S = make_case(M + N + K, M, N, K, gs)
+        A[min(3, M - 1), :gs] = 0.0
+        A[0, gs // 2] = 1e30  # an overflowing group: scale inf
+        got = q.linear_i8(dev(A), dev(W), dev(S), gs)
+        assert_bits(got, orc.linear(A, W, S, gs), f"{M}x{N}x{K} gs {gs}")
+
+
+@pytest.mark.parametrize("gs", [32, 64, 128])
+@pytest.mark.parametrize("M,N", [(9, 70), (70, 11001), (70, 17003)], ids=str)
+def test_swiglu_tiles(orc, M, N, gs):
+    K = 640 if gs == 128 else 320
+    A, Wg, Sg = make_case(M + N, M, N, K, gs)
+    _, Wu, Su = make_case(M + N + 1, M, N, K, gs)
+    got = q.linear_i8_swiglu(dev(A), dev(Wg), dev(Sg), dev(Wu), dev(Su), gs)
+    want = orc.swiglu(orc.linear(A, Wg, Sg, gs), orc.linear(A, Wu, Su, gs))
+    assert_bits(got, want, f"swiglu {M}x{N}x{K} gs {gs}")
+
+
+@pytest.mark.parametrize("gs", [32, 64, 128])
+@pytest.mark.parametrize("M,H,I", [(9, 128, 128), (37, 640, 384), (70, 128, 11008), (70, 128, 17024), (130, 192, 320)],
+                         ids=str)
+def test_mlp_tiles(orc, M, H, I, gs):
+    if H % gs or I % gs:
+        pytest.skip("not whole groups")
+    A, Wg, Sg = make_case(M + I, M, I, H, gs)
+    _, Wu, Su = make_case(M + I + 1, M, I, H, gs)
+    _, Wd, Sd = make_case(M + I + 2, M, H, I, gs)
+    ws = torch.zeros(q.mlp_workspace_bytes(M, H, I, gs), dtype=torch.uint8, device="cuda")
+    got = q.mlp_i8(dev(A), dev(Wg), dev(Sg), dev(Wu), dev(Su), dev(Wd), dev(Sd), gs, workspace=ws)
+    h = orc.swiglu(orc.linear(A, Wg, Sg, gs), orc.linear(A, Wu, Su, gs)).reshape(M, I)
+    assert_bits(got, orc.linear(h, Wd, Sd, gs), f"mlp {M}x{H}x{I} gs {gs}")
+
+
+@pytest.mark.parametrize("gs", [32, 64, 128])
+@pytest.mark.parametrize("M,V", [(9, 1030), (70, 6001), (70, 14003), (70, 20005)], ids=str)
+def test_argmax_tiles(orc, M, V, gs):
+    K = 128 if gs == 128 else 64
+    A, W, S = make_case(M + V, M, V, K, gs)
+    W[V - 1], S[V - 1] = W[V // 2], S[V // 2]  # a tie across blocks: the lower index wins
+    logits = torch.zeros((M, V), device="cuda")
+    ids = q.lm_head_argmax(dev(A), dev(W), dev(S), gs, logits=logits)
+    want = orc.linear(A, W, S, gs)
+    assert_bits(logits, want, "logits")
+    np.testing.assert_array_equal(ids.cpu().numpy(), orc.argmax_rows(want))
+    ids2 = q.lm_head_argmax(dev(A), dev(W), dev(S), gs) if M > 8 else ids
+    np.testing.assert_array_equal(ids2.cpu().numpy(), ids.cpu().numpy())
