@@ -174,6 +174,19 @@ bool gemv_path_ok(size_t M, size_t K, size_t gs) {
     return M <= 8 && K % 16 == 0 && K / 16 <= 512 && gs_ok_gemv(gs);
 }
 
+GemmSkinnyArgs skinny_args(const float *A, const _Float16 *Af, const float *asf, int nseg, const int8_t *const *W,
+                           const float *const *S, float *const *C, const size_t *Ns, size_t M, size_t K) {
+    GemmSkinnyArgs g{};
+    g.A = A;
+    g.Af = Af;
+    g.asf = asf;
+    for (int i = 0; i < nseg; ++i) g.seg[i] = {W[i], S[i], C[i], (int)Ns[i]};
+    g.nseg = nseg;
+    g.M = (int)M;
+    g.K = (int)K;
+    return g;
+}
+
 // Shared-activation runner: segments ride one GEMV launch (M <= 8) or one
 // quantization followed by one GEMM per segment (M > 8).
 int run_linear(const float *A, int nseg, const int8_t *const *W, const float *const *S,
@@ -210,7 +223,34 @@ int run_linear(const float *A, int nseg, const int8_t *const *W, const float *co
         if (rc) return rc;
         for (int i = 0; wide_mf && i < nseg; ++i) wide_mf = K % 512 == 0;
     }
-    if (gemv_path_ok(M, K, gs) && !wide_mf) {
+    // 2..16 rows (plain; 2..8 under SwiGLU): the split-K MFMA kernel, which
+    // quantizes the activations itself. Above 8 rows that pays while a CU gets
+    // one block of it (9..16 rows x 6144 columns: 11.5 us against 9.3 with a
+    // quantizer launch ahead; x 2048: 6.3 against 7.0).
+    bool groups = false;
+    size_t tiles = 0;
+    for (int i = 0; i < nseg; ++i) {
+        groups = groups || (G && G[i]);
+        tiles += (Ns[i] + 15) / 16;
+    }
+    const bool swiglu = mode == GEMV_SWIGLU;
+    if (!groups && mode != GEMV_ARGMAX && !wide_mf && tiles <= 0x7fffffff && K <= 0x7fffffff &&
+        gemm_skinny_serves((int)M, (int)K, (int)gs, true, swiglu)) {
+        int cus = 0;
+        rc = device_cus(&cus);
+        if (rc) return rc;
+        if (M <= 8 || tiles <= (size_t)cus) {
+            Q3VL_HIP(launch_gemm_skinny(skinny_args(A, nullptr, nullptr, nseg, W, S, C, Ns, M, K), (int)gs, swiglu, st),
+                     "skinny gemm launch");
+            return Q3VL_OK;
+        }
+    }
+    // ... and past its LDS (K > 4096 at 5..8 rows) its fragment form, where the
+    // workspace holds the fragments
+    const bool skinny_frag = !groups && mode == GEMV_PLAIN && !wide_mf && M > 4 && K <= 0x7fffffff &&
+                             gemm_skinny_serves((int)M, (int)K, (int)gs, false, false) &&
+                             (!ws || wsb >= layout(M > 8 ? M : 9, Nmax, K, gs).total);
+    if (gemv_path_ok(M, K, gs) && !wide_mf && !skinny_frag) {
         // Lane numerics apply per segment shape; segments sharing one launch
         // must agree on the path.
         const bool lanes = q3vl_uses_lane_path(M, Ns[0], K);
@@ -308,6 +348,11 @@ int run_linear(const float *A, int nseg, const int8_t *const *W, const float *co
             return Q3VL_OK;
         }
         Q3VL_HIP(launch_quantize_t16(A, aq, asT, (int)M, (int)K, (int)gs, st), "quantize launch");
+        if (skinny_frag) {
+            Q3VL_HIP(launch_gemm_skinny(skinny_args(nullptr, aq, asT, nseg, W, S, C, Ns, M, K), (int)gs, false, st),
+                     "skinny gemm launch");
+            return Q3VL_OK;
+        }
         if (mode == GEMV_SWIGLU) {
             GemmT16Args g{aq, asT, Mt, W[0], S[0], W[1], S[1], C[0], (int)M, (int)Ns[0], (int)K};
             Q3VL_HIP(launch_gemm_t16(g, (int)gs, true, cus, st), "gemm launch");
@@ -710,6 +755,11 @@ int q3vl_mlp_i8(const float *A, const int8_t *Wg, const float *Sg, const int8_t 
         gu.hq = hq;
         gu.hqs = hs;
         Q3VL_HIP(launch_gemm_t16(gu, gs, true, cus, st), "gate|up gemm launch");
+        if (gemm_skinny_serves((int)M, (int)I, gs, false, false)) {
+            Q3VL_HIP(launch_gemm_skinny(skinny_args(nullptr, hq, hs, 1, &Wd, &Sd, &Y, &H, M, I), gs, false, st),
+                     "down gemm launch");
+            return Q3VL_OK;
+        }
         GemmT16Args dn{hq, hs, Mt, Wd, Sd, nullptr, nullptr, Y, (int)M, (int)H, (int)I};
         Q3VL_HIP(launch_gemm_t16(dn, gs, false, cus, st), "down gemm launch");
         return Q3VL_OK;

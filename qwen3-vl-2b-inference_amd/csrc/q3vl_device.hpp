@@ -138,6 +138,15 @@ Q3VL_INLINE void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// Order this wave's LDS accesses before and after it, so that lanes may read
+// what other lanes of the wave wrote: the wave's LDS operations execute in
+// order, so no instruction is needed, but the compiler has to keep the order.
+Q3VL_INLINE void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Group scale from the 16 per-lane partial sums of squares of one group
 // (i8:148-152): the caller passes the sum tree already reduced; this applies
 // rms = sqrt(sumsq/gs + 1e-6), s = rms * fp32(1/127).

@@ -151,6 +151,26 @@ bool gemm_t16_serves(int M, int N, int K, int gs);
 int gemm_t16_argmax_cols(int M, int N, int gs, int cus);
 hipError_t launch_gemm_t16(const GemmT16Args &a, int gs, bool swiglu, int cus, hipStream_t st);
 
+// 2..16 rows against up to three weights (group size 64 or 128, K a multiple
+// of 128 up to 6144): K split over a block's waves, the ordered sums after.
+// The activations either as fp32 (quantized inside) or, A null, as
+// launch_quantize_t16's fragments. swiglu (2..8 rows, fp32): segments 0 and 1
+// are gate and up, H goes to segment 0's C.
+struct GemmSkinnyArgs {
+    const float *A;
+    const _Float16 *Af;
+    const float *asf;
+    struct {
+        const int8_t *W;
+        const float *S;
+        float *C;
+        int N;
+    } seg[3];
+    int nseg, M, K;
+};
+bool gemm_skinny_serves(int M, int K, int gs, bool fp32, bool swiglu);
+hipError_t launch_gemm_skinny(const GemmSkinnyArgs &a, int gs, bool swiglu, hipStream_t st);
+
 // 16 or fewer rows of fp32 activations A [M, K] against a wide weight (K %
 // 512 == 0, K <= 2048): quantized inside the kernel, 16 x 16 MFMA tiles with
 // the weights loaded straight into the operands. With argmax partial buffers

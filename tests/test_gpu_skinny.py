@@ -1,0 +1,76 @@
+"""GPU parity of the few-row split-K GEMM (csrc/gemm_skinny.hip): each row
+padding (4, 8, 16) and activation form (fp32 quantized inside, fragments), the
+piece counts per wave at their edges (K of one 128-byte piece up to 6144),
+ragged columns, segments, and the SwiGLU form. Against the CPU oracle, bit for
+bit (the products and the ordered sums round as the oracle's)."""
+import numpy as np
+import pytest
+
+from golden.gen import make_case
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+import q3vl_int8 as q  # noqa: E402
+
+
+def dev(a):
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def assert_bits(got, want, what):
+    torch.cuda.synchronize()
+    g, w = got.cpu().numpy().view(np.uint32), np.ascontiguousarray(want, np.float32).view(np.uint32)
+    bad = np.flatnonzero(g.ravel() != w.ravel())
+    assert bad.size == 0, f"{what}: {bad.size} of {g.size} differ, first at {bad[:5]}"
+
+
+@pytest.mark.parametrize("gs", [64, 128])
+@pytest.mark.parametrize("K", [128, 896, 1024, 1152, 2048, 3072, 4096, 5120, 6144])
+def test_linear_few_rows(orc, K, gs):
+    for M, N in ((2, 33), (4, 70), (5, 16), (8, 50), (9, 47), (16, 70)):
+        A, W, S = make_case(M + N + K, M, N, K, gs)
+        A[M - 1, :gs] = 0.0
+        A[0, gs - 1] = 1e30  # an overflowing group: scale inf
+        assert_bits(q.linear_i8(dev(A), dev(W), dev(S), gs), orc.linear(A, W, S, gs), f"{M}x{N}x{K} gs {gs}")
+
+
+@pytest.mark.parametrize("M", [3, 8, 16])
+def test_multi_few_rows(orc, M):
+    K, gs, Ns = 1152, 64, (33, 16, 50)
+    cases = [make_case(M + n, M, n, K, gs) for n in Ns]
+    A = cases[0][0]
+    outs = q.linear_i8_multi(dev(A), [dev(w) for _, w, _ in cases], [dev(s) for _, _, s in cases], gs)
+    for o, (_, w, s), n in zip(outs, cases, Ns):
+        assert_bits(o, orc.linear(A, w, s, gs), f"segment of {n}")
+
+
+@pytest.mark.parametrize("gs", [64, 128])
+@pytest.mark.parametrize("M,N,K", [(2, 33, 128), (4, 70, 2048), (7, 40, 1152), (8, 100, 2048), (3, 20, 3072)], ids=str)
+def test_swiglu_few_rows(orc, M, N, K, gs):
+    A, Wg, Sg = make_case(M + N, M, N, K, gs)
+    _, Wu, Su = make_case(M + N + 1, M, N, K, gs)
+    got = q.linear_i8_swiglu(dev(A), dev(Wg), dev(Sg), dev(Wu), dev(Su), gs)
+    assert_bits(got, orc.swiglu(orc.linear(A, Wg, Sg, gs), orc.linear(A, Wu, Su, gs)), f"swiglu {M}x{N}x{K} gs {gs}")
+
+
+@pytest.mark.parametrize("gs", [64, 128])
+@pytest.mark.parametrize("M,H,I", [(2, 256, 384), (8, 1024, 6144), (13, 128, 6144), (16, 256, 256)], ids=str)
+def test_mlp_few_rows(orc, M, H, I, gs):
+    A, Wg, Sg = make_case(M + I, M, I, H, gs)
+    _, Wu, Su = make_case(M + I + 1, M, I, H, gs)
+    _, Wd, Sd = make_case(M + I + 2, M, H, I, gs)
+    ws = torch.zeros(q.mlp_workspace_bytes(M, H, I, gs), dtype=torch.uint8, device="cuda")
+    got = q.mlp_i8(dev(A), dev(Wg), dev(Sg), dev(Wu), dev(Su), dev(Wd), dev(Sd), gs, workspace=ws)
+    h = orc.swiglu(orc.linear(A, Wg, Sg, gs), orc.linear(A, Wu, Su, gs)).reshape(M, I)
+    assert_bits(got, orc.linear(h, Wd, Sd, gs), f"mlp {M}x{H}x{I} gs {gs}")
+
+
+def test_small_workspace_still_served(orc):
+    """5..8 rows at K = 6144 with a workspace too small for the fragments: the
+    integer GEMV, as before."""
+    M, N, K = 6, 40, 6144
+    A, W, S = make_case(5, M, N, K, 64)
+    small = torch.zeros(2 * 8192 * M * 4 + 512, dtype=torch.uint8, device="cuda")  # the argmax partials alone
+    assert small.numel() < q.workspace_bytes(M, N, K, 64)
+    assert_bits(q.linear_i8(dev(A), dev(W), dev(S), 64, workspace=small), orc.linear(A, W, S, 64), "small workspace")
