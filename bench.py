@@ -872,7 +872,7 @@ def pmc_workload_gemm():
 def pmc_workload_lmhead():
     """Workload for the lm_head traffic passes: the calibration copy of
     pmc_workload, then 3 calls each of config 3's lm_head + argmax at M = 1
-    (gemv_kernel) and M = 8 (gemm_mf_wide_kernel), every call on its own
+    (gemv_kernel) and M = 8 (gemm_wide_kernel), every call on its own
     weight copy (3 x 331 MB: each streams from HBM)."""
     import torch
     import q3vl_int8 as q

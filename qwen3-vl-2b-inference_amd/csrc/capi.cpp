@@ -210,18 +210,28 @@ int run_linear(const float *A, int nseg, const int8_t *const *W, const float *co
     int rc = resolve_ws(ws, wsb, L.total, &wbase);
     if (rc) return rc;
 
-    // 5..8 rows against a very wide weight (the lm_head over a batch of
-    // rows): the MFMA kernels below (16-row tiles, see wide16) stream the
-    // weights faster than the general GEMV's integer dot products.
-    bool wide_mf = M >= 5 && M <= 8 && gs == 64 && mode != GEMV_SWIGLU;
-    for (int i = 0; wide_mf && i < nseg; ++i)
-        wide_mf = !(G && G[i]) && (size_t)Ns[i] * K >= ((size_t)1 << 26) &&
-                  (size_t)Ns[i] * K <= 0x7fffffffULL;
-    if (wide_mf) {
+    // 2..16 rows against a very wide weight (the lm_head over a batch of
+    // rows): MFMA tiles that read the weights once, quantizing inside.
+    bool wide = mode != GEMV_SWIGLU && M <= 16;
+    for (int i = 0; wide && i < nseg; ++i)
+        wide = !(G && G[i]) && (size_t)Ns[i] * K >= ((size_t)1 << 26) &&
+               gemm_wide_serves((int)M, (int)Ns[i], (int)K, (int)gs);
+    if (wide) {
         int cus = 0;
         rc = device_cus(&cus);
         if (rc) return rc;
-        for (int i = 0; wide_mf && i < nseg; ++i) wide_mf = K % 512 == 0;
+        for (int i = 0; i < nseg; ++i) {
+            const bool am = mode == GEMV_ARGMAX;
+            float *pv = am ? reinterpret_cast<float *>(wbase + L.parts_val) : nullptr;
+            int32_t *pi = am ? reinterpret_cast<int32_t *>(wbase + L.parts_idx) : nullptr;
+            const int nparts = gemm_wide_parts((int)Ns[i], cus);
+            if ((size_t)nparts > kMaxGemvParts)
+                return fail(Q3VL_ERR_UNSUPPORTED, "argmax: %d partials exceed %zu", nparts, kMaxGemvParts);
+            Q3VL_HIP(launch_gemm_wide(A, W[i], S[i], C[i], (int)M, (int)Ns[i], (int)K, (int)gs, pv, pi, cus, st),
+                     "wide gemm launch");
+            if (am) Q3VL_HIP(launch_argmax_final(pv, pi, nparts, (int)M, ids, st), "argmax launch");
+        }
+        return Q3VL_OK;
     }
     // 2..16 rows (plain; 2..8 under SwiGLU): the split-K MFMA kernel, which
     // quantizes the activations itself. Above 8 rows that pays while a CU gets
@@ -234,7 +244,7 @@ int run_linear(const float *A, int nseg, const int8_t *const *W, const float *co
         tiles += (Ns[i] + 15) / 16;
     }
     const bool swiglu = mode == GEMV_SWIGLU;
-    if (!groups && mode != GEMV_ARGMAX && !wide_mf && tiles <= 0x7fffffff && K <= 0x7fffffff &&
+    if (!groups && mode != GEMV_ARGMAX && tiles <= 0x7fffffff && K <= 0x7fffffff &&
         gemm_skinny_serves((int)M, (int)K, (int)gs, true, swiglu)) {
         int cus = 0;
         rc = device_cus(&cus);
@@ -247,10 +257,10 @@ int run_linear(const float *A, int nseg, const int8_t *const *W, const float *co
     }
     // ... and past its LDS (K > 4096 at 5..8 rows) its fragment form, where the
     // workspace holds the fragments
-    const bool skinny_frag = !groups && mode == GEMV_PLAIN && !wide_mf && M > 4 && K <= 0x7fffffff &&
+    const bool skinny_frag = !groups && mode == GEMV_PLAIN && M > 4 && K <= 0x7fffffff &&
                              gemm_skinny_serves((int)M, (int)K, (int)gs, false, false) &&
                              (!ws || wsb >= layout(M > 8 ? M : 9, Nmax, K, gs).total);
-    if (gemv_path_ok(M, K, gs) && !wide_mf && !skinny_frag) {
+    if (gemv_path_ok(M, K, gs) && !skinny_frag) {
         // Lane numerics apply per segment shape; segments sharing one launch
         // must agree on the path.
         const bool lanes = q3vl_uses_lane_path(M, Ns[0], K);
@@ -320,33 +330,6 @@ int run_linear(const float *A, int nseg, const int8_t *const *W, const float *co
     }
     if (use_t16) {
         const int Mt = (int)((M + 31) / 32);
-        // 5..16 rows against a very wide weight (the lm_head over a batch of
-        // rows): 16-row MFMA tiles with the weights loaded straight into the
-        // operands, the activations quantized inside the kernel
-        bool wide16 = Mt == 1 && M >= 5 && gs == 64 && K % 512 == 0 && mode != GEMV_SWIGLU;
-        for (int i = 0; wide16 && i < nseg; ++i)
-            wide16 = (size_t)Ns[i] * K >= ((size_t)1 << 26) &&
-                     gemm_mf_wide_serves((int)M, (int)Ns[i], (int)K);
-        if (wide16) {
-            for (int i = 0; i < nseg; ++i) {
-                float *pv = nullptr;
-                int32_t *pi = nullptr;
-                int nparts = 0;
-                if (mode == GEMV_ARGMAX) {
-                    pv = reinterpret_cast<float *>(wbase + LG.parts_val);
-                    pi = reinterpret_cast<int32_t *>(wbase + LG.parts_idx);
-                    nparts = gemm_mf_wide_parts((int)Ns[i], cus);
-                    if ((size_t)nparts > kMaxGemvParts)
-                        return fail(Q3VL_ERR_UNSUPPORTED, "argmax: %d partials exceed %zu", nparts,
-                                    kMaxGemvParts);
-                }
-                Q3VL_HIP(launch_gemm_mf_wide(A, W[i], S[i], C[i], (int)M, (int)Ns[i], (int)K, pv, pi, cus, st),
-                         "wide gemm launch");
-                if (mode == GEMV_ARGMAX)
-                    Q3VL_HIP(launch_argmax_final(pv, pi, nparts, (int)M, ids, st), "argmax launch");
-            }
-            return Q3VL_OK;
-        }
         Q3VL_HIP(launch_quantize_t16(A, aq, asT, (int)M, (int)K, (int)gs, st), "quantize launch");
         if (skinny_frag) {
             Q3VL_HIP(launch_gemm_skinny(skinny_args(nullptr, aq, asT, nseg, W, S, C, Ns, M, K), (int)gs, false, st),

@@ -31,7 +31,7 @@
 //   fragments of quantize_t16_kernel.
 #include "q3vl_device.hpp"
 #include "q3vl_kernels.hpp"
-#include "q3vl_quant_team.hpp"
+#include "q3vl_mfma.hpp"
 
 namespace q3vl {
 

@@ -37,7 +37,7 @@
 
 #include "q3vl_device.hpp"
 #include "q3vl_kernels.hpp"
-#include "q3vl_quant_team.hpp"
+#include "q3vl_mfma.hpp"
 
 namespace q3vl {
 
@@ -101,36 +101,6 @@ hipError_t launch_quantize_t16(const float *A, _Float16 *qf, float *asf, int M, 
 }
 
 // ---------------------------------------------------------------- the GEMM
-// Loads with an LDS destination: lane l's 16 (4) bytes at voff + soff of the
-// resource go to LDS at lds + 16 l (4 l). Written in asm because the compiler
-// would wait for every such load before any later LDS read; dma_wait<N>()
-// waits until at most N of this wave's loads are in flight (they complete in
-// order).
-typedef uint32_t rsrc_t __attribute__((ext_vector_type(4)));
-Q3VL_INLINE rsrc_t make_rsrc(const void *p, uint32_t bytes) {
-    const uint64_t a = (uint64_t)p;
-    return (rsrc_t){(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a),
-                    (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32)),
-                    (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000u};
-}
-Q3VL_INLINE void dma16(rsrc_t r, int voff, int soff, int lds) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                 :: "s"(lds), "v"(voff), "s"(r), "s"(soff) : "memory");
-#endif
-}
-Q3VL_INLINE void dma4(rsrc_t r, int voff, int soff, int lds) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds"
-                 :: "s"(lds), "v"(voff), "s"(r), "s"(soff) : "memory");
-#endif
-}
-template <int N> Q3VL_INLINE void dma_wait() {
-#if defined(__HIP_DEVICE_COMPILE__)
-    asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N < 63 ? N : 63) : "memory");  // (the counter's field)
-#endif
-}
-
 // The tile shape. GS: group size. A: 16-row tiles of the block (2, 4 or 8:
 // all of its waves share its rows). B: 16-column tiles of a wave (SwiGLU: B/2
 // gate, B/2 up). NW: waves, side by side along the columns. A unit is UC

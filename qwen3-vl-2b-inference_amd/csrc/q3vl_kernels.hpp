@@ -171,14 +171,13 @@ struct GemmSkinnyArgs {
 bool gemm_skinny_serves(int M, int K, int gs, bool fp32, bool swiglu);
 hipError_t launch_gemm_skinny(const GemmSkinnyArgs &a, int gs, bool swiglu, hipStream_t st);
 
-// 16 or fewer rows of fp32 activations A [M, K] against a wide weight (K %
-// 512 == 0, K <= 2048): quantized inside the kernel, 16 x 16 MFMA tiles with
-// the weights loaded straight into the operands. With argmax partial buffers
-// it leaves gemm_mf_wide_parts(N, cus) partials per row, [parts][M]; C may
-// then be null.
-bool gemm_mf_wide_serves(int M, int N, int K);
-int gemm_mf_wide_parts(int N, int cus);
-hipError_t launch_gemm_mf_wide(const float *A, const int8_t *W, const float *S, float *C, int M, int N,
-                               int K, float *part_val, int32_t *part_idx, int cus, hipStream_t st);
+// 2..16 rows of fp32 activations A [M, K] against a wide weight (K % 256 ==
+// 0, within the block's LDS): quantized inside the kernel, 16 x 16 MFMA tiles.
+// With argmax partial buffers it leaves gemm_wide_parts(N, cus) partials per
+// row, [parts][M]; C may then be null.
+bool gemm_wide_serves(int M, int N, int K, int gs);
+int gemm_wide_parts(int N, int cus);
+hipError_t launch_gemm_wide(const float *A, const int8_t *W, const float *S, float *C, int M, int N, int K, int gs,
+                            float *part_val, int32_t *part_idx, int cus, hipStream_t st);
 
 }  // namespace q3vl

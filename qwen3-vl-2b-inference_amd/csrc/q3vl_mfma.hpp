@@ -1,6 +1,6 @@
-// q3vl_quant_team.hpp -- device pieces the MFMA kernels share: the activation
-// quantizer of one (row, group) by a quad of lanes, and the widening of int8
-// weights to fp16.
+// q3vl_mfma.hpp -- device pieces the MFMA kernels share: the activation
+// quantizer of one (row, group) by a quad of lanes, the widening of int8
+// weights to fp16, and loads with an LDS destination.
 #pragma once
 
 #include "q3vl_device.hpp"
@@ -83,6 +83,43 @@ Q3VL_INLINE half8_t widen8(uint32_t x, uint32_t y) {
     widen4(x, a, b);
     widen4(y, c, d);
     return __builtin_bit_cast(half8_t, (u32x4){a, b, c, d});
+}
+
+// Loads with an LDS destination: lane l's 16 (4) bytes at voff + soff of the
+// resource go to LDS at lds + 16 l (4 l). Written in asm because the compiler
+// would wait for every such load before any later LDS read; dma_wait<N>()
+// waits until at most N of this wave's loads are in flight (they complete in
+// order).
+typedef uint32_t rsrc_t __attribute__((ext_vector_type(4)));
+Q3VL_INLINE rsrc_t make_rsrc(const void *p, uint32_t bytes) {
+    const uint64_t a = (uint64_t)p;
+    return (rsrc_t){(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a),
+                    (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32)),
+                    (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000u};
+}
+Q3VL_INLINE void dma16(rsrc_t r, int voff, int soff, int lds) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                 :: "s"(lds), "v"(voff), "s"(r), "s"(soff) : "memory");
+#endif
+}
+// (the same for bytes read once: kept out of the caches' way)
+Q3VL_INLINE void dma16_nt(rsrc_t r, int voff, int soff, int lds) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds"
+                 :: "s"(lds), "v"(voff), "s"(r), "s"(soff) : "memory");
+#endif
+}
+Q3VL_INLINE void dma4(rsrc_t r, int voff, int soff, int lds) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds"
+                 :: "s"(lds), "v"(voff), "s"(r), "s"(soff) : "memory");
+#endif
+}
+template <int N> Q3VL_INLINE void dma_wait() {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("s_waitcnt vmcnt(%0)" :: "n"(N < 63 ? N : 63) : "memory");  // (the counter's field)
+#endif
 }
 
 }  // namespace q3vl

@@ -74,3 +74,22 @@ def test_small_workspace_still_served(orc):
     small = torch.zeros(2 * 8192 * M * 4 + 512, dtype=torch.uint8, device="cuda")  # the argmax partials alone
     assert small.numel() < q.workspace_bytes(M, N, K, 64)
     assert_bits(q.linear_i8(dev(A), dev(W), dev(S), 64, workspace=small), orc.linear(A, W, S, 64), "small workspace")
+
+
+# the wide kernel (csrc/gemm_wide.hip): N * K >= 2^26, each row padding and
+# group size, with fewer tiles than waves and more, ragged rows
+@pytest.mark.parametrize("gs", [32, 64, 128])
+@pytest.mark.parametrize("M,V,K", [(2, 65541, 1024), (4, 32801, 2048), (7, 131075, 512), (9, 262150, 256), (16, 33003, 2048)],
+                         ids=str)
+def test_wide_few_rows(orc, M, V, K, gs):
+    A, W, S = make_case(M + V, M, V, K, gs)
+    W[V - 1], S[V - 1] = W[V // 2], S[V // 2]  # a tie across waves: the lower index wins
+    A[0, 1] = 1e30  # an overflowing group: scale inf
+    want = orc.linear(A, W, S, gs)
+    logits = torch.zeros((M, V), device="cuda")
+    ids = q.lm_head_argmax(dev(A), dev(W), dev(S), gs, logits=logits)
+    assert_bits(logits, want, f"logits {M}x{V}x{K} gs {gs}")
+    np.testing.assert_array_equal(ids.cpu().numpy(), orc.argmax_rows(want))
+    if M <= 8:  # without stored logits
+        np.testing.assert_array_equal(q.lm_head_argmax(dev(A), dev(W), dev(S), gs).cpu().numpy(), ids.cpu().numpy())
+    assert_bits(q.linear_i8(dev(A), dev(W), dev(S), gs), want, "plain")
