@@ -525,11 +525,14 @@ __global__ __launch_bounds__(64 * T::NW, MINB) void gemm_t16_kernel(
 #pragma unroll
         for (int i = 0; i < A; ++i)
 #pragma unroll
-            for (int j = 0; j < NJ; ++j)
+            for (int j = 0; j < NJ; ++j) {
+                const float gv[4] = {out[i][j][0], out[i][j][1], out[i][j][2], out[i][j][3]};
+                const float uv[4] = {out[i][j + NJ][0], out[i][j + NJ][1], out[i][j + NJ][2], out[i][j + NJ][3]};
+                float h[4];
+                silu_mul_n<4>(gv, uv, h);
 #pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    ht[(16 * i + 4 * c + e) * HLD + 16 * (wid * NJ + j) + nl] =
-                        silu_mul(out[i][j][e], out[i][j + NJ][e]);
+                for (int e = 0; e < 4; ++e) ht[(16 * i + 4 * c + e) * HLD + 16 * (wid * NJ + j) + nl] = h[e];
+            }
         lds_barrier();
         constexpr int GB = COLS / GS;  // groups of the tile
         for (int p = tid; p < 16 * A * GB * 4; p += NT) {
@@ -601,6 +604,19 @@ __global__ __launch_bounds__(64 * T::NW, MINB) void gemm_t16_kernel(
 
     // ---- store (an argmax caller that wants no logits passes C = null)
     if (!args.C) return;  // uniform
+    if constexpr (SWIGLU) {
+#pragma unroll
+        for (int i = 0; i < A; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                const float gv[4] = {out[i][j][0], out[i][j][1], out[i][j][2], out[i][j][3]};
+                const float uv[4] = {out[i][j + NJ][0], out[i][j + NJ][1], out[i][j + NJ][2], out[i][j + NJ][3]};
+                float h[4];
+                silu_mul_n<4>(gv, uv, h);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) out[i][j][e] = h[e];
+            }
+    }
 #pragma unroll
     for (int i = 0; i < A; ++i)
 #pragma unroll
@@ -611,8 +627,7 @@ __global__ __launch_bounds__(64 * T::NW, MINB) void gemm_t16_kernel(
             for (int j = 0; j < NJ; ++j) {
                 const int col = n0 + 16 * (wid * NJ + j) + nl;
                 if (col < N)
-                    args.C[(size_t)mrow * N + col] = SWIGLU ? silu_mul(out[i][j][e], out[i][SWIGLU ? j + NJ : j][e])
-                                                            : out[i][j][e];
+                    args.C[(size_t)mrow * N + col] = out[i][j][e];
             }
         }
 }

@@ -82,3 +82,20 @@ def test_argmax_tiles(orc, M, V, gs):
     np.testing.assert_array_equal(ids.cpu().numpy(), orc.argmax_rows(want))
     ids2 = q.lm_head_argmax(dev(A), dev(W), dev(S), gs) if M > 8 else ids
     np.testing.assert_array_equal(ids2.cpu().numpy(), ids.cpu().numpy())
+
+
+@pytest.mark.parametrize("M", [1, 4, 40], ids=str)
+def test_silu_range(orc, M):
+    """Gates from 2^-75 to past expf's range on both sides, 0, infinite and
+    NaN: the SwiGLU epilogues' fast division and its other case."""
+    N, K, gs = 320, 64, 64
+    A, Wg, Sg = make_case(7, M, N, K, gs)
+    _, Wu, Su = make_case(8, M, N, K, gs)
+    Sg[:, 0] = np.exp2(np.linspace(-75, 12, N)).astype(np.float32)
+    Sg[5:9, 0] = 0.0, np.inf, 1e37, np.nan
+    got = q.linear_i8_swiglu(dev(A), dev(Wg), dev(Sg), dev(Wu), dev(Su), gs)
+    want = orc.swiglu(orc.linear(A, Wg, Sg, gs), orc.linear(A, Wu, Su, gs)).reshape(M, N)
+    torch.cuda.synchronize()
+    g, ok = got.cpu().numpy().reshape(M, N), ~np.isnan(want)
+    np.testing.assert_array_equal(np.isnan(g), ~ok)
+    np.testing.assert_array_equal(g[ok].view(np.uint32), want[ok].view(np.uint32))
