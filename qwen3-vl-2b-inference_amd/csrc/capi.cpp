@@ -320,7 +320,7 @@ int run_linear(const float *A, int nseg, const int8_t *const *W, const float *co
         // a vocabulary of more partials than the workspace holds: refused at
         // group size 64, scanned from stored logits at the others
         const size_t cols = gs == 64 && K % 512 == 0 && M > 32
-                                ? 64 : (size_t)gemm_t16_argmax_cols((int)M, (int)Ns[0], (int)gs, cus);
+                                ? 64 : (size_t)gemm_t16_argmax_cols((int)M, (int)Ns[0], (int)K, (int)gs, cus);
         const size_t nparts = (Ns[0] + cols - 1) / cols;
         if (nparts > kMaxGemvParts) {
             if (gs == 64 && K % 512 == 0)
@@ -349,7 +349,7 @@ int run_linear(const float *A, int nseg, const int8_t *const *W, const float *co
                 // logits are stored only when the caller asked for them
                 g.part_val = reinterpret_cast<float *>(wbase + LG.parts_val);
                 g.part_idx = reinterpret_cast<int32_t *>(wbase + LG.parts_idx);
-                const int cols = gemm_t16_argmax_cols((int)M, (int)Ns[i], (int)gs, cus);
+                const int cols = gemm_t16_argmax_cols((int)M, (int)Ns[i], (int)K, (int)gs, cus);
                 nparts = (int)((Ns[i] + cols - 1) / cols);
             }
             Q3VL_HIP(launch_gemm_t16(g, (int)gs, false, cus, st), "gemm launch");

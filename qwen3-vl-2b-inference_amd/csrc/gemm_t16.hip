@@ -647,42 +647,79 @@ static hipError_t launch_t16(const GemmT16Args &a, hipStream_t st) {
     return hipGetLastError();
 }
 
-// Which tile, from timings on MI355X (us a GEMM, weights rotating through
-// more than the L2s; a unit is one group of 64). The fixed cost of a unit in
-// a block falls with the tile (a 32 x 128 block takes 0.29 us a unit, 64 x 128
-// 0.45, or 0.73 for two blocks on a CU, 128 x 128 0.65), so a product too
-// small to give every CU a block runs the fewest rows a block, and a large
-// one the tile whose rounds over the device cost least:
-// * 32 x 64 while its blocks fit the CUs: 64 x 2048 x 2048 8.4 (32 x 128:
-//   9.8; the 32 x 32-tile GEMM before it 14.5);
-// * 32 x 128 while its blocks fit: 512 x 2048 x 6144 27.5 (64 x 128: 44; 42
-//   before), 784 x 1024 x 4096 18.9 (31; 32 before);
-// * then 64 x 128 or 128 x 128: 1000 x 2048 x 6144 48 (128 x 128: 63), 1501 x
-//   2048 x 6144 65 (64 x 128: 70; 92 before).
-// SwiGLU (output columns; each has a gate and an up column): 32 x 64 up to two
-// blocks a CU (64 x 6144 x 2048: 14.5, 64 x 64: 21), 64 x 128 while its blocks
-// fit the CUs (300 rows: 31, 128 x 128: 44; 43 before), else 128 x 128 (1501
-// rows: 132, 64 x 128: 136; 149 before). At group 128 the tiles hold 128
-// columns (whole groups of the h they quantize) and at most 64 rows (more
-// spill).
-static int t16_tile(int M, int N, int gs, bool swiglu, int cus) {
-    auto blocks = [&](int r, int c) { return (long)((M + r - 1) / r) * ((N + c - 1) / c); };
-    if (swiglu) {
-        if (gs == 128) return blocks(32, 128) <= cus ? 0 : 1;
-        if (blocks(32, 64) <= 2L * cus) return 0;
-        return blocks(64, 128) <= cus ? 1 : 2;
+// Which tile, from timings on MI355X (us; weights rotating through more than
+// the L2s; a unit is one group of 64). A tile's blocks run in rounds of `cap`
+// blocks a CU, a round costs fix + unit * K / 64, and the product takes the
+// tile whose rounds cost least: one too small to give every CU a block runs
+// the fewest rows a block, a large one the tile with the least work a row.
+// * plain, 32 x 64: 64 x 2048 x 2048 8.4 us (32 x 128: 9.8; the 32 x 32-tile
+//   GEMM before: 14.5); 32 x 128: 512 x 2048 x 6144 27.5 (64 x 128: 44; 42
+//   before); 64 x 128, two blocks a CU: 1000 x 2048 x 6144 48 (128 x 128: 63);
+//   128 x 128: 1501 x 2048 x 6144 65 (64 x 128: 70; 92 before);
+// * SwiGLU (output columns; each has a gate and an up column), 32 x 64, two
+//   blocks a CU: 64 x 6144 x 2048 14.5 (64 x 64: 21); 64 x 128: 300 rows 31
+//   (128 x 128: 44; 43 before); 128 x 128: 512 rows 47 (64 x 128: 59; 52
+//   before). At group 128 the tiles hold 128 columns (whole groups of the h
+//   they quantize) and at most 64 rows (more spill).
+// A large product's last round is often nearly empty (1501 x 6144 SwiGLU: 576
+// blocks, 2.25 rounds): the rows of the whole rounds then run first, and the
+// rest as a product of its own, with its own tile, where the sum of the two
+// and another launch cost less (the MLP block of 1501 x 2048 x 6144: 189 us,
+// 200 in one product).
+struct T16Tile {
+    int rows, cols, cap;  // cap: blocks a CU
+    float unit, fix;
+};
+struct T16Plan {
+    int tile, rows, tile2;  // rows 0..rows-1 by tile, the others (if any) by tile2
+};
+static const T16Tile kPlain[4] = {{32, 64, 1, 0.21f, 2}, {32, 128, 1, 0.27f, 2}, {64, 128, 2, 0.75f, 3}, {128, 128, 1, 0.65f, 3}};
+static const T16Tile kSwiglu[3] = {{32, 64, 2, 0.36f, 7}, {64, 128, 1, 0.69f, 8}, {128, 128, 1, 1.09f, 9}};
+static const T16Tile kSwiglu128[2] = {{32, 128, 1, 0.60f, 8}, {64, 128, 1, 0.65f, 8}};
+
+static T16Plan t16_plan(int M, int N, int K, int gs, bool swiglu, bool argmax, int cus) {
+    const T16Tile *tiles = !swiglu ? kPlain : gs == 128 ? kSwiglu128 : kSwiglu;
+    const int n = !swiglu ? 4 : gs == 128 ? 2 : 3;
+    auto cost = [&](int t, int m) {
+        const T16Tile &q = tiles[t];
+        const long blocks = (long)((m + q.rows - 1) / q.rows) * ((N + q.cols - 1) / q.cols);
+        // (of two blocks a CU, the second costs about two thirds of the first)
+        const long slots = (long)q.cap * cus, rounds = (blocks + slots - 1) / slots;
+        const long last = blocks - (rounds - 1) * slots;
+        const float part = q.cap == 2 && last <= cus ? 0.62f : 1.0f;
+        return ((float)(rounds - 1) + part) * (q.fix + q.unit * (float)K / 64);
+    };
+    T16Plan best{0, M, 0};
+    float least = 1e30f;
+    for (int t = 0; t < n; ++t) {
+        const float c = cost(t, M);
+        if (c < least) {
+            least = c;
+            best = {t, M, 0};
+        }
     }
-    if (blocks(32, 64) <= cus) return 0;
-    if (blocks(32, 128) <= cus) return 1;
-    const long b2 = blocks(64, 128);
-    const long c2 = b2 <= cus ? 45 : (b2 + 2 * cus - 1) / (2 * cus) * 73;
-    const long c3 = (blocks(128, 128) + cus - 1) / cus * 65;
-    return c2 <= c3 ? 2 : 3;
+    if (argmax) return best;  // (one set of partials)
+    const T16Tile &big = tiles[n - 1];
+    const long nb = (N + big.cols - 1) / big.cols;
+    for (int r = 1; r <= 64; ++r) {  // r whole rounds of the largest tile
+        const long m1 = (long)r * cus / nb * big.rows;
+        if (m1 <= 0) continue;
+        if (m1 >= M) break;
+        const float c1 = cost(n - 1, (int)m1) + 2;
+        for (int t = 0; t < n; ++t) {
+            const float c = c1 + cost(t, M - (int)m1);
+            if (c < least) {
+                least = c;
+                best = {n - 1, (int)m1, t};
+            }
+        }
+    }
+    return best;
 }
 
 // Columns per argmax partial of a plain product.
-int gemm_t16_argmax_cols(int M, int N, int gs, int cus) {
-    return t16_tile(M, N, gs, false, cus) == 0 ? 64 : 128;
+int gemm_t16_argmax_cols(int M, int N, int K, int gs, int cus) {
+    return kPlain[t16_plan(M, N, K, gs, false, true, cus).tile].cols;
 }
 
 // The kernel addresses a block's rows with 32-bit byte offsets.
@@ -691,14 +728,13 @@ bool gemm_t16_serves(int M, int N, int K, int gs) {
            N >= 1;
 }
 
-template <int GS> static hipError_t launch_gs(const GemmT16Args &a, bool swiglu, int cus, hipStream_t st) {
-    const int tile = t16_tile(a.M, a.N, GS, swiglu, cus);
+template <int GS> static hipError_t launch_tile(const GemmT16Args &a, bool swiglu, int tile, hipStream_t st) {
     constexpr int S4 = GS == 128 ? 2 : 4;  // a stage of 256 k (the loads of more do not fit the counter)
     if (swiglu) {
         constexpr int NW = GS == 128 ? 8 : 4;
         using T0 = T16<GS, 2, 2, NW, 2, 2, true>;
         using T1 = T16<GS, 4, 2, 8, 1, 2, true>;
-        using T2 = T16<GS, GS == 128 ? 4 : 8, 2, 8, 1, 2, true>;
+        using T2 = T16<GS, GS == 128 ? 4 : 8, 2, 8, 1, 2, true>;  // (not planned at group 128)
         if (a.hq)
             return tile == 0 ? launch_t16<T0, 8 / NW, true>(a, st)
                              : tile == 1 ? launch_t16<T1, 1, true>(a, st) : launch_t16<T2, 1, true>(a, st);
@@ -709,6 +745,25 @@ template <int GS> static hipError_t launch_gs(const GemmT16Args &a, bool swiglu,
     if (tile == 1) return launch_t16<T16<GS, 2, 1, 8, S4, 2, false>, 1>(a, st);
     if (tile == 2) return launch_t16<T16<GS, 4, 1, 8, 1, 2, false>, 2>(a, st);
     return launch_t16<T16<GS, 8, 1, 8, 1, 2, false>, 1>(a, st);
+}
+
+template <int GS> static hipError_t launch_gs(const GemmT16Args &a, bool swiglu, int cus, hipStream_t st) {
+    const T16Plan p = t16_plan(a.M, a.N, a.K, GS, swiglu, a.part_val != nullptr, cus);
+    if (p.rows >= a.M) return launch_tile<GS>(a, swiglu, p.tile, st);
+    GemmT16Args x = a, y = a;  // (p.rows: whole 32-row m-tiles)
+    x.M = p.rows;
+    x.Mt = p.rows / 32;
+    y.M = a.M - p.rows;
+    y.Mt = a.Mt - x.Mt;
+    y.Af += (size_t)p.rows * a.K;
+    y.asf += (size_t)p.rows * (a.K / GS);
+    if (a.C) y.C += (size_t)p.rows * a.N;
+    if (a.hq) {
+        y.hq += (size_t)p.rows * a.N;
+        y.hqs += (size_t)p.rows * (a.N / GS);
+    }
+    const hipError_t e = launch_tile<GS>(x, swiglu, p.tile, st);
+    return e != hipSuccess ? e : launch_tile<GS>(y, swiglu, p.tile2, st);
 }
 
 hipError_t launch_gemm_t16(const GemmT16Args &a, int gs, bool swiglu, int cus, hipStream_t st) {

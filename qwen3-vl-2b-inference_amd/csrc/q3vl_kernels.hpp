@@ -148,7 +148,7 @@ hipError_t launch_quantize_t16(const float *A, _Float16 *qf, float *asf, int M, 
 // with launch_quantize_f16).
 bool gemm_t16_serves(int M, int N, int K, int gs);
 // Columns per argmax partial of a plain product.
-int gemm_t16_argmax_cols(int M, int N, int gs, int cus);
+int gemm_t16_argmax_cols(int M, int N, int K, int gs, int cus);
 hipError_t launch_gemm_t16(const GemmT16Args &a, int gs, bool swiglu, int cus, hipStream_t st);
 
 // 2..16 rows against up to three weights (group size 64 or 128, K a multiple

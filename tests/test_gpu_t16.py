@@ -99,3 +99,24 @@ def test_silu_range(orc, M):
     g, ok = got.cpu().numpy().reshape(M, N), ~np.isnan(want)
     np.testing.assert_array_equal(np.isnan(g), ~ok)
     np.testing.assert_array_equal(g[ok].view(np.uint32), want[ok].view(np.uint32))
+
+
+@pytest.mark.parametrize("gs", [32, 64, 128])
+@pytest.mark.parametrize("M", [641, 700, 2100], ids=str)
+def test_row_split(orc, M, gs):
+    """A nearly empty last round runs as a product of its own: 640 + 1 and
+    640 + 60 rows of a SwiGLU pair, the same in front of down (group 32 and
+    64), and 2048 + 52 rows of a plain product."""
+    if M == 2100:
+        A, W, S = make_case(M, M, 2048, 512, gs)
+        assert_bits(q.linear_i8(dev(A), dev(W), dev(S), gs), orc.linear(A, W, S, gs), f"plain gs {gs}")
+        return
+    H, I = 128, 6144
+    A, Wg, Sg = make_case(M, M, I, H, gs)
+    _, Wu, Su = make_case(M + 1, M, I, H, gs)
+    _, Wd, Sd = make_case(M + 2, M, H, I, gs)
+    h = orc.swiglu(orc.linear(A, Wg, Sg, gs), orc.linear(A, Wu, Su, gs)).reshape(M, I)
+    assert_bits(q.linear_i8_swiglu(dev(A), dev(Wg), dev(Sg), dev(Wu), dev(Su), gs), h, f"swiglu gs {gs}")
+    ws = torch.zeros(q.mlp_workspace_bytes(M, H, I, gs), dtype=torch.uint8, device="cuda")
+    got = q.mlp_i8(dev(A), dev(Wg), dev(Sg), dev(Wu), dev(Su), dev(Wd), dev(Sd), gs, workspace=ws)
+    assert_bits(got, orc.linear(h, Wd, Sd, gs), f"mlp gs {gs}")
