@@ -133,40 +133,51 @@ template <int GS_, int A_, int B_, int NW_, int SU_, int NB_, bool SWIGLU_> stru
     static_assert(!SWIGLU || B % 2 == 0, "gate and up tiles");
     static_assert(SU >= CB && 4 % SU == 0 && NA * 1024 * NW == ABUF && SBUF <= 1024 * NW, "stages");
     static_assert(LDS <= 160 * 1024, "LDS");
-    // Loads that a wave issues between the load a wait is for and the wait, in
-    // the loop's steady state: 'a' the activation stage met at unit us, 'b'
-    // the weight stage first read in unit us, 'w' the next body's w_s. (The
-    // loop is entered with nothing in flight, so its first turns wait for no
-    // less.)
+    // Which loads go out in unit u of the K loop (before its first unit: as
+    // units -8 .. -1 would issue them, for the stages there are): the next
+    // stage but one of the activations where unit u first reads the next, the
+    // next body but one's w_s at a body's start, the weight stage that takes
+    // the slot consumed at the unit's end. Stages below 0: none.
+    static constexpr int fdiv(int a, int b) { return (a + 64 * b) / b - 64; }
+    static constexpr int a_stage(int u) { return (u + 64) % SU == SU - CB ? fdiv(u, SU) + 2 : -1; }
+    static constexpr int w_body(int u) { return (u + 64) % 4 == 0 ? fdiv(u, 4) + 2 : -1; }
+    static constexpr int b_stage(int u) { return (u + 65) % UB == UB - 1 ? fdiv(u + 1, UB) + NB : -1; }
+    // Loads that a wave issues between the load a wait is for and the wait, the
+    // least over the first bodies and the steady state: 'a' the activation
+    // stage met at unit us, 'b' the weight stage first read in unit us, 'w'
+    // the next body's w_s; 's' the loop's start, where the first stage of each
+    // (and as many activations as the first fragments reach) have landed.
     static constexpr int behind(char what, int us) {
-        int n = 0, at = -1;  // loads issued so far; count right behind the one waited for
-        for (int pass = 0; pass < 2; ++pass) {
-            n = 0;
-            int target_a = -1, target_b = -1, target_w = -1;
-            // the wait's place: body 5, unit us; what it waits for
-            if (what == 'a') target_a = (20 + us) / SU + 1;
-            if (what == 'b') target_b = (20 + us + 1) / UB;
-            if (what == 'w') target_w = 6;
-            for (int u = 0; u < 24; ++u) {
-                const int su = u % SU;
-                if (su == SU - CB) {
-                    if (pass == 1 && what == 'a' && u == 20 + us) return n - at;
+        int least = 1 << 30;
+        for (int body = 0; body < 6; ++body) {
+            int n = 0, at = -1;
+            const int end = 4 * body + us;  // the wait's unit
+            for (int u = -8; u <= end; ++u) {
+                if (what == 's' && u == 0) break;
+                if (what == 'a' && u == end) break;
+                if (a_stage(u) >= 0) {
                     n += NA + 1;
-                    if (u / SU + 2 == target_a) at = n;
+                    if (what == 'a' ? a_stage(u) == end / SU + 1 : what == 's' && a_stage(u) <= (PD - 1) / (A * SU)) at = n;
                 }
-                if (u % 4 == 0) {
+                if (w_body(u) >= 0) {
                     n += B * WST;
-                    if (u / 4 + 2 == target_w) at = n;
+                    if (what == 'w' ? w_body(u) == body + 1 : what == 's' && w_body(u) == 0) at = n;
                 }
-                if ((u + 1) % UB == 0 && pass == 1 && what == 'b' && u == 20 + us) return n - at;
-                if ((u + 1) % UB == UB - 1) {
+                if (what == 'b' && u == end) break;
+                if (b_stage(u) >= 0 && !(what == 's' && b_stage(u) >= NB)) {
                     n += 2 * B;
-                    if ((u + 1) / UB + NB == target_b) at = n;
+                    if (what == 'b' ? b_stage(u) == (end + 1) / UB : what == 's' && b_stage(u) == 0) at = n;
                 }
-                if (u % 4 == 3 && pass == 1 && what == 'w' && u == 23) return n - at;
             }
+            least = at < 0 ? -1 : n - at < least ? n - at : least;
+            if (at < 0) break;
         }
-        return 0;
+        return least;
+    }
+    static constexpr bool waits() {  // every wait's load is among those before it
+        for (int us = 0; us < 4; ++us)
+            if ((a_stage(us) >= 0 && behind('a', us) < 0) || ((us + 1) % UB == 0 && behind('b', us) < 0)) return false;
+        return behind('w', 3) >= 0 && behind('s', 0) >= 0;
     }
 };
 
@@ -427,13 +438,14 @@ __global__ __launch_bounds__(64 * T::NW, MINB) void gemm_t16_kernel(
     static_assert(2 * SU > SU - 1 + (A - 1 + PD) / A, "fragments are read at most one stage ahead");
 
     if (nbody > 0) {
-        load_a(0, 0);
-        load_a(1, min(1, lasta));
+        static_assert(T::waits(), "loads");
 #pragma unroll
-        for (int x = 0; x < NB; ++x) load_b(x, min(x, lastb));
-        load_ws(0, 0);
-        load_ws(1, min(1, nbody - 1));
-        dma_wait<0>();
+        for (int u = -8; u < 0; ++u) {  // (slot: the stage's number; one past the slots goes out below)
+            if (T::a_stage(u) >= 0) load_a(T::a_stage(u), min(T::a_stage(u), lasta));
+            if (T::w_body(u) >= 0) load_ws(T::w_body(u), min(T::w_body(u), nbody - 1));
+            if (T::b_stage(u) >= 0 && T::b_stage(u) < NB) load_b(T::b_stage(u), min(T::b_stage(u), lastb));
+        }
+        dma_wait<T::behind('s', 0)>();
         lds_barrier();
         read_ws(0);
         read_as(0, 0, 0);
@@ -647,52 +659,76 @@ static hipError_t launch_t16(const GemmT16Args &a, hipStream_t st) {
     return hipGetLastError();
 }
 
-// Which tile, from timings on MI355X (us; weights rotating through more than
-// the L2s; a unit is one group of 64). A tile's blocks run in rounds of `cap`
-// blocks a CU, a round costs fix + unit * K / 64, and the product takes the
-// tile whose rounds cost least: one too small to give every CU a block runs
-// the fewest rows a block, a large one the tile with the least work a row.
-// * plain, 32 x 64: 64 x 2048 x 2048 8.4 us (32 x 128: 9.8; the 32 x 32-tile
-//   GEMM before: 14.5); 32 x 128: 512 x 2048 x 6144 27.5 (64 x 128: 44; 42
-//   before); 64 x 128, two blocks a CU: 1000 x 2048 x 6144 48 (128 x 128: 63);
-//   128 x 128: 1501 x 2048 x 6144 65 (64 x 128: 70; 92 before);
-// * SwiGLU (output columns; each has a gate and an up column), 32 x 64, two
-//   blocks a CU: 64 x 6144 x 2048 14.5 (64 x 64: 21); 64 x 128: 300 rows 31
-//   (128 x 128: 44; 43 before); 128 x 128: 512 rows 47 (64 x 128: 59; 52
-//   before). At group 128 the tiles hold 128 columns (whole groups of the h
-//   they quantize) and at most 64 rows (more spill).
+// Which tile. A tile's blocks run in rounds of `cap` blocks a CU; a round of
+// L blocks a CU takes fix + unit[L - 1] * K / 64 us (measured on MI355X at
+// group 64, weights rotating through more than the L2s; group 32 takes 1.15
+// to 1.25 times as long in every tile). The product takes the tile whose
+// rounds cost least. Small products want one small block on every CU, larger
+// ones two or three blocks of 64 x 64, which wait at barriers of their own
+// (4 waves each), and where those leave a round half empty, larger blocks:
+// * plain (us; 32 x 64 / 32 x 128 / 64 x 64 / 64 x 128 / 128 x 128):
+//     196 x 2048 x 4096   14.7 /  -   /  -   /  -   /  -
+//     512 x 2048 x 6144   30.5 / 26.9 / 39.6 / 43.5 / 63
+//     784 x 3072 x 1024   17.3 / 18.2 / 13.6 / 15.5 / 15.9
+//     784 x 4096 x 1024    -   /  -   / 18.0 / 16.3 / 16.6
+//     1000 x 2048 x 6144  65.5 / 54.9 / 46.3 / 48.0 / 65.6
+//     1501 x 2048 x 6144   -   /  -   / 66.8 / 71.4 / 69.4
+//     1501 x 4096 x 2048   -   /  -   / 47.1 / 44.1 / 52.8
+//   and at group 128 1501 x 2048 x 6144 68 / 71 / 58 (64 x 64, 64 x 128, 128 x 128);
+// * SwiGLU (output columns, each a gate and an up column; 32 x 64 / 64 x 64 /
+//   128 x 128), N = 6144, K = 2048: 16 rows 12.7 / 19.7 / 41.7, 200 rows 28.0
+//   / 27.5 / 43.2, 300 rows 36.3 / 28.8 / -, 512 rows - / 45.8 / 48.3, 1501
+//   rows 166 / 130 / 131. Up to one block a CU the 32 x 64 tile takes longer
+//   stages of activations (12.7 us, 13.3 without). At group 128 a tile has
+//   128 columns (whole groups of the h it quantizes) and at most 64 rows
+//   (more spill): 300 rows 31 (32 x 128), 26 (64 x 128).
 // A large product's last round is often nearly empty (1501 x 6144 SwiGLU: 576
-// blocks, 2.25 rounds): the rows of the whole rounds then run first, and the
-// rest as a product of its own, with its own tile, where the sum of the two
-// and another launch cost less (the MLP block of 1501 x 2048 x 6144: 189 us,
-// 200 in one product).
+// blocks of 128 x 128, 2.25 rounds): the rows of the whole rounds then run
+// first, and the rest as a product of its own, with its own tile, where the
+// two and another launch cost less (at 1501 rows 88 us + 27 in place of 130).
 struct T16Tile {
-    int rows, cols, cap;  // cap: blocks a CU
-    float unit, fix;
+    int rows, cols, cap;
+    float unit[3], fix;
 };
 struct T16Plan {
-    int tile, rows, tile2;  // rows 0..rows-1 by tile, the others (if any) by tile2
+    int tile, rows, tile2;  // rows 0 .. rows - 1 by tile, the others (if any) by tile2
 };
-static const T16Tile kPlain[4] = {{32, 64, 1, 0.21f, 2}, {32, 128, 1, 0.27f, 2}, {64, 128, 2, 0.75f, 3}, {128, 128, 1, 0.65f, 3}};
-static const T16Tile kSwiglu[3] = {{32, 64, 2, 0.36f, 7}, {64, 128, 1, 0.69f, 8}, {128, 128, 1, 1.09f, 9}};
-static const T16Tile kSwiglu128[2] = {{32, 128, 1, 0.60f, 8}, {64, 128, 1, 0.65f, 8}};
+enum { P32x64, P32x128, P64x64, P64x128, P128x128, PLAIN_TILES };
+static const T16Tile kPlain[PLAIN_TILES] = {{32, 64, 1, {0.20f}, 2},
+                                            {32, 128, 1, {0.26f}, 2},
+                                            {64, 64, 3, {0.34f, 0.43f, 0.65f}, 5},
+                                            {64, 128, 2, {0.43f, 0.67f}, 6},
+                                            {128, 128, 1, {0.66f}, 5.5f}};
+static const T16Tile kPlain128[PLAIN_TILES] = {{32, 64, 1, {0.16f}, 2},
+                                               {32, 128, 1, {0.21f}, 2},
+                                               {64, 64, 3, {0.21f, 0.40f, 0.66f}, 5},
+                                               {64, 128, 2, {0.29f, 0.68f}, 6},
+                                               {128, 128, 1, {0.56f}, 5}};
+enum { S32x64L, S32x64, S64x64, S128x128, SWIGLU_TILES };
+static const T16Tile kSwiglu[SWIGLU_TILES] = {{32, 64, 1, {0.18f}, 7},
+                                              {32, 64, 2, {0.20f, 0.36f}, 7},
+                                              {64, 64, 2, {0.35f, 0.61f}, 7.5f},
+                                              {128, 128, 1, {1.16f}, 9}};
+enum { S32x128, S64x128, SWIGLU128_TILES };
+static const T16Tile kSwiglu128[SWIGLU128_TILES] = {{32, 128, 1, {0.25f}, 8}, {64, 128, 1, {0.55f}, 8}};
 
 static T16Plan t16_plan(int M, int N, int K, int gs, bool swiglu, bool argmax, int cus) {
-    const T16Tile *tiles = !swiglu ? kPlain : gs == 128 ? kSwiglu128 : kSwiglu;
-    const int n = !swiglu ? 4 : gs == 128 ? 2 : 3;
-    auto cost = [&](int t, int m) {
-        const T16Tile &q = tiles[t];
+    const T16Tile *tiles = swiglu ? (gs == 128 ? kSwiglu128 : kSwiglu) : gs == 128 ? kPlain128 : kPlain;
+    const int n = swiglu ? (gs == 128 ? (int)SWIGLU128_TILES : (int)SWIGLU_TILES) : (int)PLAIN_TILES;
+    const float units = (float)K / 64;
+    auto cost = [&](const T16Tile &q, int m) {
         const long blocks = (long)((m + q.rows - 1) / q.rows) * ((N + q.cols - 1) / q.cols);
-        // (of two blocks a CU, the second costs about two thirds of the first)
-        const long slots = (long)q.cap * cus, rounds = (blocks + slots - 1) / slots;
-        const long last = blocks - (rounds - 1) * slots;
-        const float part = q.cap == 2 && last <= cus ? 0.62f : 1.0f;
-        return ((float)(rounds - 1) + part) * (q.fix + q.unit * (float)K / 64);
+        const long slots = (long)q.cap * cus, rounds = (blocks - 1) / slots;
+        const long level = (blocks - rounds * slots - 1) / cus;  // of the last round
+        return (float)rounds * (q.fix + q.unit[q.cap - 1] * units) + q.fix + q.unit[level] * units;
     };
     T16Plan best{0, M, 0};
     float least = 1e30f;
     for (int t = 0; t < n; ++t) {
-        const float c = cost(t, M);
+        // (the 64-column tiles leave twice the argmax partials: only where
+        // they are few)
+        if (argmax && tiles[t].cols == 64 && (long)((M + 31) / 32) * ((N + 63) / 64) > cus) continue;
+        const float c = cost(tiles[t], M);
         if (c < least) {
             least = c;
             best = {t, M, 0};
@@ -701,13 +737,13 @@ static T16Plan t16_plan(int M, int N, int K, int gs, bool swiglu, bool argmax, i
     if (argmax) return best;  // (one set of partials)
     const T16Tile &big = tiles[n - 1];
     const long nb = (N + big.cols - 1) / big.cols;
-    for (int r = 1; r <= 64; ++r) {  // r whole rounds of the largest tile
+    for (int r = 1; r <= 16; ++r) {  // r whole rounds of the largest tile
         const long m1 = (long)r * cus / nb * big.rows;
-        if (m1 <= 0) continue;
         if (m1 >= M) break;
-        const float c1 = cost(n - 1, (int)m1) + 2;
+        if (m1 <= 0) continue;
+        const float c1 = cost(big, (int)m1) + 2;
         for (int t = 0; t < n; ++t) {
-            const float c = c1 + cost(t, M - (int)m1);
+            const float c = c1 + cost(tiles[t], M - (int)m1);
             if (c < least) {
                 least = c;
                 best = {n - 1, (int)m1, t};
@@ -719,7 +755,7 @@ static T16Plan t16_plan(int M, int N, int K, int gs, bool swiglu, bool argmax, i
 
 // Columns per argmax partial of a plain product.
 int gemm_t16_argmax_cols(int M, int N, int K, int gs, int cus) {
-    return kPlain[t16_plan(M, N, K, gs, false, true, cus).tile].cols;
+    return kPlain[t16_plan(M, N, K, gs, false, true, cus).tile].cols;  // (the same at every group size)
 }
 
 // The kernel addresses a block's rows with 32-bit byte offsets.
@@ -728,23 +764,32 @@ bool gemm_t16_serves(int M, int N, int K, int gs) {
            N >= 1;
 }
 
-template <int GS> static hipError_t launch_tile(const GemmT16Args &a, bool swiglu, int tile, hipStream_t st) {
+template <int GS> static hipError_t launch_plain(const GemmT16Args &a, int tile, hipStream_t st) {
     constexpr int S4 = GS == 128 ? 2 : 4;  // a stage of 256 k (the loads of more do not fit the counter)
-    if (swiglu) {
-        constexpr int NW = GS == 128 ? 8 : 4;
-        using T0 = T16<GS, 2, 2, NW, 2, 2, true>;
-        using T1 = T16<GS, 4, 2, 8, 1, 2, true>;
-        using T2 = T16<GS, GS == 128 ? 4 : 8, 2, 8, 1, 2, true>;  // (not planned at group 128)
-        if (a.hq)
-            return tile == 0 ? launch_t16<T0, 8 / NW, true>(a, st)
-                             : tile == 1 ? launch_t16<T1, 1, true>(a, st) : launch_t16<T2, 1, true>(a, st);
-        return tile == 0 ? launch_t16<T0, 8 / NW>(a, st)
-                         : tile == 1 ? launch_t16<T1, 1>(a, st) : launch_t16<T2, 1>(a, st);
-    }
-    if (tile == 0) return launch_t16<T16<GS, 2, 1, 4, S4, 3, false>, 1>(a, st);
-    if (tile == 1) return launch_t16<T16<GS, 2, 1, 8, S4, 2, false>, 1>(a, st);
-    if (tile == 2) return launch_t16<T16<GS, 4, 1, 8, 1, 2, false>, 2>(a, st);
+    // (four waves: two blocks' worth of registers, or the sums would move
+    // through accumulation registers, 16.5 us instead of 14.7 at 196 x 2048 x 4096)
+    if (tile == P32x64) return launch_t16<T16<GS, 2, 1, 4, S4, 3, false>, 2>(a, st);
+    if (tile == P32x128) return launch_t16<T16<GS, 2, 1, 8, S4, 2, false>, 1>(a, st);
+    if (tile == P64x64) return launch_t16<T16<GS, 4, 1, 4, 1, 2, false>, 3>(a, st);
+    if (tile == P64x128) return launch_t16<T16<GS, 4, 1, 8, 1, 2, false>, 2>(a, st);
     return launch_t16<T16<GS, 8, 1, 8, 1, 2, false>, 1>(a, st);
+}
+
+template <int GS, bool HQ> static hipError_t launch_swiglu(const GemmT16Args &a, int tile, hipStream_t st) {
+    if constexpr (GS == 128) {
+        if (tile == S32x128) return launch_t16<T16<GS, 2, 2, 8, 2, 2, true>, 1, HQ>(a, st);
+        return launch_t16<T16<GS, 4, 2, 8, 1, 2, true>, 1, HQ>(a, st);
+    } else {
+        if (tile == S32x64L) return launch_t16<T16<GS, 2, 2, 4, 4, 2, true>, 2, HQ>(a, st);
+        if (tile == S32x64) return launch_t16<T16<GS, 2, 2, 4, 2, 2, true>, 2, HQ>(a, st);
+        if (tile == S64x64) return launch_t16<T16<GS, 4, 2, 4, 1, 2, true>, 2, HQ>(a, st);
+        return launch_t16<T16<GS, 8, 2, 8, 1, 2, true>, 1, HQ>(a, st);
+    }
+}
+
+template <int GS> static hipError_t launch_tile(const GemmT16Args &a, bool swiglu, int tile, hipStream_t st) {
+    if (!swiglu) return launch_plain<GS>(a, tile, st);
+    return a.hq ? launch_swiglu<GS, true>(a, tile, st) : launch_swiglu<GS, false>(a, tile, st);
 }
 
 template <int GS> static hipError_t launch_gs(const GemmT16Args &a, bool swiglu, int cus, hipStream_t st) {

@@ -25,9 +25,10 @@ def assert_bits(got, want, what):
     assert bad.size == 0, f"{what}: {bad.size} of {g.size} differ, first at {bad[:5]}"
 
 
-# rows x columns that reach the four plain tiles on 256 CUs (32 x 64, 32 x
-# 128, 64 x 128, 128 x 128), each with ragged last tiles
-PLAIN = [(9, 70), (33, 130), (70, 6001), (70, 14003), (70, 20005), (131, 12801)]
+# rows x columns that reach the five plain tiles on 256 CUs (32 x 64, 32 x
+# 128, 64 x 64, 64 x 128, 128 x 128), each with ragged last tiles
+PLAIN = [(9, 70), (33, 130), (70, 6001), (70, 14003), (70, 20005), (131, 12801), (70, 21851), (131, 16571),
+         (131, 19871), (70, 24821)]
 
 
 @pytest.mark.parametrize("gs", [32, 64, 128])
@@ -44,7 +45,7 @@ def test_linear_tiles(orc, M, N, gs):
 
 
 @pytest.mark.parametrize("gs", [32, 64, 128])
-@pytest.mark.parametrize("M,N", [(9, 70), (70, 11001), (70, 17003)], ids=str)
+@pytest.mark.parametrize("M,N", [(9, 70), (9, 16571), (40, 16571), (70, 11001), (70, 17003)], ids=str)
 def test_swiglu_tiles(orc, M, N, gs):
     K = 640 if gs == 128 else 320
     A, Wg, Sg = make_case(M + N, M, N, K, gs)
@@ -55,7 +56,8 @@ def test_swiglu_tiles(orc, M, N, gs):
 
 
 @pytest.mark.parametrize("gs", [32, 64, 128])
-@pytest.mark.parametrize("M,H,I", [(9, 128, 128), (37, 640, 384), (70, 128, 11008), (70, 128, 17024), (130, 192, 320)],
+@pytest.mark.parametrize("M,H,I", [(9, 128, 128), (37, 640, 384), (70, 128, 11008), (70, 128, 17024), (130, 192, 320),
+                                   (9, 128, 16640), (40, 128, 16640)],
                          ids=str)
 def test_mlp_tiles(orc, M, H, I, gs):
     if H % gs or I % gs:
