@@ -136,8 +136,9 @@ template <int GS_, int A_, int B_, int NW_, int SU_, int NB_, bool SWIGLU_> stru
     // Which loads go out in unit u of the K loop (before its first unit: as
     // units -8 .. -1 would issue them, for the stages there are): the next
     // stage but one of the activations where unit u first reads the next, the
-    // next body but one's w_s at a body's start, the weight stage that takes
-    // the slot consumed at the unit's end. Stages below 0: none.
+    // next body but one's w_s in a body's first unit (after the wait for the
+    // weights), the weight stage that takes the slot consumed at the unit's
+    // end. Stages below 0: none.
     static constexpr int fdiv(int a, int b) { return (a + 64 * b) / b - 64; }
     static constexpr int a_stage(int u) { return (u + 64) % SU == SU - CB ? fdiv(u, SU) + 2 : -1; }
     static constexpr int w_body(int u) { return (u + 64) % 4 == 0 ? fdiv(u, 4) + 2 : -1; }
@@ -159,11 +160,11 @@ template <int GS_, int A_, int B_, int NW_, int SU_, int NB_, bool SWIGLU_> stru
                     n += NA + 1;
                     if (what == 'a' ? a_stage(u) == end / SU + 1 : what == 's' && a_stage(u) <= (PD - 1) / (A * SU)) at = n;
                 }
+                if (what == 'b' && u == end) break;
                 if (w_body(u) >= 0) {
                     n += B * WST;
                     if (what == 'w' ? w_body(u) == body + 1 : what == 's' && w_body(u) == 0) at = n;
                 }
-                if (what == 'b' && u == end) break;
                 if (b_stage(u) >= 0 && !(what == 's' && b_stage(u) >= NB)) {
                     n += 2 * B;
                     if (what == 'b' ? b_stage(u) == (end + 1) / UB : what == 's' && b_stage(u) == 0) at = n;
@@ -390,7 +391,6 @@ __global__ __launch_bounds__(64 * T::NW, MINB) void gemm_t16_kernel(
             load_a(b2, min(n / SU + 2, lasta));
             __builtin_amdgcn_sched_barrier(0);
         }
-        if constexpr (us == 0) load_ws((n >> 2) & 1, min((n >> 2) + 2, nbody - 1));
         if constexpr ((us + 1) % UB == 0) dma_wait<T::behind('b', us)>();
         read_raw(sb, (us + 1) % UB);
         __builtin_amdgcn_sched_barrier(0);
@@ -416,6 +416,18 @@ __global__ __launch_bounds__(64 * T::NW, MINB) void gemm_t16_kernel(
                 }
                 __builtin_amdgcn_sched_barrier(0);
                 fold(i, us, k, tt, ws);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (us == 0 && i == 0) {
+                // this body's w_s (read at the last one's end) are in their
+                // registers: before that their slot must not be refilled, and
+                // nothing else orders the refill behind the reads. By now the
+                // wait costs nothing; at the unit's start it would.
+#pragma unroll
+                for (int j = 0; j < B; ++j)
+#pragma unroll
+                    for (int k = 0; k < NG; ++k) asm volatile("" ::"v"(ws[j][k]));
+                load_ws((n >> 2) & 1, min((n >> 2) + 2, nbody - 1));
                 __builtin_amdgcn_sched_barrier(0);
             }
             if (i + 2 == A && (us + 1) % UB == UB - 1) {  // the slot is consumed
