@@ -237,32 +237,33 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(GemmSkinnyArgs a) {
     }
 }
 
+// Rows the quantizer pads to (0: fragments), and the 128-byte pieces a wave
+// takes at most: what fits the LDS at every group size. One table for what is
+// served and for the kernels there are.
+static int skinny_rw(int M, bool fp32) { return !fp32 ? 0 : M <= 4 ? 4 : M <= 8 ? 8 : 16; }
+static constexpr int skinny_pieces(int rw, bool swiglu) { return swiglu || rw == 16 ? 3 : rw == 8 ? 4 : 6; }
+
 // LDS of a block: weights (then products), w_s, and the quantized rows.
-static size_t skinny_lds(int M, int K, int gs, bool fp32, bool swiglu) {
-    const size_t rw = M <= 4 ? 4 : M <= 8 ? 8 : 16, kg = K / gs;
-    return (swiglu ? 2 : 1) * ((size_t)K * 16 + kg * 64) + (fp32 ? 2 * K * rw + kg * 64 : 0);
+static constexpr size_t skinny_lds(int rw, int K, int gs, bool swiglu) {
+    const size_t kg = K / gs;
+    return (swiglu ? 2 : 1) * ((size_t)K * 16 + kg * 64) + (rw ? (size_t)2 * K * rw + kg * 64 : 0);
 }
 
 template <int GS, int NP, int RW, bool SW> static hipError_t launch_one(const GemmSkinnyArgs &a, int grid, hipStream_t st) {
     static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_skinny_kernel<GS, NP, RW, SW>),
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     if (attr != hipSuccess) return attr;
-    gemm_skinny_kernel<GS, NP, RW, SW><<<grid, 512, skinny_lds(a.M, a.K, GS, RW > 0, SW), st>>>(a);
+    gemm_skinny_kernel<GS, NP, RW, SW><<<grid, 512, skinny_lds(RW, a.K, GS, SW), st>>>(a);
     return hipGetLastError();
 }
 
-template <int GS, int RW, bool SW> static hipError_t launch_np(const GemmSkinnyArgs &a, int grid, hipStream_t st) {
-    const int np = (a.K / 128 + 7) / 8;  // 128-byte pieces per wave
-    if constexpr (!SW && RW <= 4) {      // (only these fit the LDS)
-        if (np == 6) return launch_one<GS, 6, RW, SW>(a, grid, st);
-        if (np == 5) return launch_one<GS, 5, RW, SW>(a, grid, st);
+template <int GS, int RW, bool SW, int NP = skinny_pieces(RW, SW)>
+static hipError_t launch_np(const GemmSkinnyArgs &a, int grid, hipStream_t st) {
+    static_assert(skinny_lds(RW, 1024 * NP, GS, SW) <= 160 * 1024, "LDS");
+    if constexpr (NP > 0) {
+        if ((a.K / 128 + 7) / 8 == NP) return launch_one<GS, NP, RW, SW>(a, grid, st);
+        return launch_np<GS, RW, SW, NP - 1>(a, grid, st);
     }
-    if constexpr (!SW && RW <= 8) {
-        if (np == 4) return launch_one<GS, 4, RW, SW>(a, grid, st);
-    }
-    if (np == 3) return launch_one<GS, 3, RW, SW>(a, grid, st);
-    if (np == 2) return launch_one<GS, 2, RW, SW>(a, grid, st);
-    if (np == 1) return launch_one<GS, 1, RW, SW>(a, grid, st);
     return hipErrorInvalidValue;
 }
 
@@ -275,8 +276,8 @@ template <int GS> static hipError_t launch_rw(const GemmSkinnyArgs &a, bool swig
 }
 
 bool gemm_skinny_serves(int M, int K, int gs, bool fp32, bool swiglu) {
-    return M >= 2 && M <= (swiglu ? 8 : 16) && (gs == 64 || gs == 128) && K > 0 && K % 128 == 0 && K <= 6144 &&
-           (fp32 || !swiglu) && skinny_lds(M, K, gs, fp32, swiglu) <= 160 * 1024;
+    return M >= 2 && M <= (swiglu ? 8 : 16) && (gs == 64 || gs == 128) && K > 0 && K % 128 == 0 && (fp32 || !swiglu) &&
+           K <= 1024 * skinny_pieces(skinny_rw(M, fp32), swiglu);
 }
 
 hipError_t launch_gemm_skinny(const GemmSkinnyArgs &a, int gs, bool swiglu, hipStream_t st) {

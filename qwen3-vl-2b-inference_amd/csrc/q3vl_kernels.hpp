@@ -152,10 +152,11 @@ int gemm_t16_argmax_cols(int M, int N, int K, int gs, int cus);
 hipError_t launch_gemm_t16(const GemmT16Args &a, int gs, bool swiglu, int cus, hipStream_t st);
 
 // 2..16 rows against up to three weights (group size 64 or 128, K a multiple
-// of 128 up to 6144): K split over a block's waves, the ordered sums after.
-// The activations either as fp32 (quantized inside) or, A null, as
-// launch_quantize_t16's fragments. swiglu (2..8 rows, fp32): segments 0 and 1
-// are gate and up, H goes to segment 0's C.
+// of 128): K split over a block's waves, the ordered sums after. The
+// activations either as fp32 (quantized inside; K up to 6144 at 2..4 rows,
+// 4096 at 5..8, 3072 at 9..16) or, A null, as launch_quantize_t16's fragments
+// (K up to 6144). swiglu (2..8 rows, fp32, K up to 3072): segments 0 and 1 are
+// gate and up, H goes to segment 0's C.
 struct GemmSkinnyArgs {
     const float *A;
     const _Float16 *Af;

@@ -35,6 +35,32 @@ def test_linear_few_rows(orc, K, gs):
         assert_bits(q.linear_i8(dev(A), dev(W), dev(S), gs), orc.linear(A, W, S, gs), f"{M}x{N}x{K} gs {gs}")
 
 
+@pytest.mark.parametrize("gs", [64, 128])
+@pytest.mark.parametrize("M,N,K", [(6, 40, 4224), (6, 40, 4608), (8, 33, 4864), (9, 47, 3200), (16, 70, 3328)], ids=str)
+def test_linear_past_the_pieces(orc, M, N, K, gs):
+    """K past the pieces a wave takes with these rows (4096 at 5..8, 3072 at
+    9..16): the fragment form."""
+    A, W, S = make_case(M + N + K, M, N, K, gs)
+    A[0, gs - 1] = 1e30
+    assert_bits(q.linear_i8(dev(A), dev(W), dev(S), gs), orc.linear(A, W, S, gs), f"{M}x{N}x{K} gs {gs}")
+
+
+@pytest.mark.parametrize("gs", [64, 128])
+@pytest.mark.parametrize("M,N,K", [(2, 33, 3200), (3, 70, 3584), (4, 40, 3840), (6, 40, 3200)], ids=str)
+def test_swiglu_past_the_pieces(orc, M, N, K, gs):
+    """K past 3072 under SwiGLU: the integer GEMV; the MLP of such a width too."""
+    A, Wg, Sg = make_case(M + N, M, N, K, gs)
+    _, Wu, Su = make_case(M + N + 1, M, N, K, gs)
+    h = orc.swiglu(orc.linear(A, Wg, Sg, gs), orc.linear(A, Wu, Su, gs))
+    assert_bits(q.linear_i8_swiglu(dev(A), dev(Wg), dev(Sg), dev(Wu), dev(Su), gs), h, f"swiglu {M}x{N}x{K} gs {gs}")
+    I = 256
+    _, Wg, Sg = make_case(M, M, I, K, gs)
+    _, Wu, Su = make_case(M + 1, M, I, K, gs)
+    _, Wd, Sd = make_case(M + 2, M, K, I, gs)
+    h = orc.swiglu(orc.linear(A, Wg, Sg, gs), orc.linear(A, Wu, Su, gs)).reshape(M, I)
+    assert_bits(q.mlp_i8(dev(A), dev(Wg), dev(Sg), dev(Wu), dev(Su), dev(Wd), dev(Sd), gs), orc.linear(h, Wd, Sd, gs), "mlp")
+
+
 @pytest.mark.parametrize("M", [3, 8, 16])
 def test_multi_few_rows(orc, M):
     K, gs, Ns = 1152, 64, (33, 16, 50)
