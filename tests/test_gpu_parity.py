@@ -330,6 +330,18 @@ def test_swiglu_dense_float_sweep(orc):
     np.testing.assert_array_equal(out[~nan].view(np.uint32), want[~nan].view(np.uint32))
 
 
+def test_swiglu_all_ones_divisor(orc):
+    """The gates about 2^-23, where 1 + expf(-g) is 2 - 2^-23 and a quotient
+    corrected with a reciprocal that is not the rounded one misses by an ulp;
+    whole waves of that gate, and it beside others."""
+    one = np.float32(2.0 ** -23).view(np.uint32)
+    bits = np.concatenate([np.full(256, one), one + np.arange(-2048, 2049),
+                           *[np.float32(2.0 ** e).view(np.uint32) + np.arange(-256, 257) for e in range(-41, -19)]])
+    g = np.concatenate([bits, bits | 0x80000000]).astype(np.uint32).view(np.float32)
+    u = np.ones_like(g)
+    assert_bits_equal(host(q.swiglu(dev(g), dev(u))), orc.swiglu(g, u), "swiglu")
+
+
 @pytest.mark.parametrize("M", [1, 8])
 def test_lm_head_argmax_parity(orc, M):
     V, K, gs = 151936, 2048, 64
