@@ -308,6 +308,12 @@ int run_linear(const float *A, int nseg, const int8_t *const *W, const float *co
     }
     _Float16 *aq = reinterpret_cast<_Float16 *>(wbase + LG.aq);
     float *asT = reinterpret_cast<float *>(wbase + LG.as);
+    if (skinny_frag) {  // (segments of no columns among them)
+        Q3VL_HIP(launch_quantize_t16(A, aq, asT, (int)M, (int)K, (int)gs, st), "quantize launch");
+        Q3VL_HIP(launch_gemm_skinny(skinny_args(nullptr, aq, asT, nseg, W, S, C, Ns, M, K), (int)gs, false, st),
+                 "skinny gemm launch");
+        return Q3VL_OK;
+    }
     // Without group sums: the fragment-order GEMM, one per segment, gate and
     // up together under SwiGLU.
     bool use_t16 = true;
@@ -331,11 +337,6 @@ int run_linear(const float *A, int nseg, const int8_t *const *W, const float *co
     if (use_t16) {
         const int Mt = (int)((M + 31) / 32);
         Q3VL_HIP(launch_quantize_t16(A, aq, asT, (int)M, (int)K, (int)gs, st), "quantize launch");
-        if (skinny_frag) {
-            Q3VL_HIP(launch_gemm_skinny(skinny_args(nullptr, aq, asT, nseg, W, S, C, Ns, M, K), (int)gs, false, st),
-                     "skinny gemm launch");
-            return Q3VL_OK;
-        }
         if (mode == GEMV_SWIGLU) {
             GemmT16Args g{aq, asT, Mt, W[0], S[0], W[1], S[1], C[0], (int)M, (int)Ns[0], (int)K};
             Q3VL_HIP(launch_gemm_t16(g, (int)gs, true, cus, st), "gemm launch");

@@ -92,6 +92,21 @@ def test_mlp_few_rows(orc, M, H, I, gs):
     assert_bits(got, orc.linear(h, Wd, Sd, gs), f"mlp {M}x{H}x{I} gs {gs}")
 
 
+@pytest.mark.parametrize("M", [6, 8, 12])
+def test_multi_empty_segment(orc, M):
+    """A segment of no columns among the others, in the fragment form (K past
+    what the rows' quantizer leaves of the LDS) as elsewhere."""
+    K, gs, Ns = 5120, 64, (33, 0, 50)
+    cases = [make_case(M + n, M, n, K, gs) if n else (None, np.zeros((0, K), np.int8), np.zeros((0, K // gs), np.float32))
+             for n in Ns]
+    A = cases[0][0]
+    ws = torch.zeros(q.workspace_bytes(M, max(Ns), K, gs), dtype=torch.uint8, device="cuda")
+    outs = q.linear_i8_multi(dev(A), [dev(w) for _, w, _ in cases], [dev(s) for _, _, s in cases], gs, workspace=ws)
+    for o, (_, w, s), n in zip(outs, cases, Ns):
+        if n:
+            assert_bits(o, orc.linear(A, w, s, gs), f"segment of {n}")
+
+
 def test_small_workspace_still_served(orc):
     """5..8 rows at K = 6144 with a workspace too small for the fragments: the
     integer GEMV, as before."""
