@@ -255,11 +255,13 @@ int run_linear(const float *A, int nseg, const int8_t *const *W, const float *co
             return Q3VL_OK;
         }
     }
-    // ... and past its LDS (K > 4096 at 5..8 rows) its fragment form, where the
-    // workspace holds the fragments
+    // ... and past its LDS (K > 4096 at 5..8 rows) its fragment form. At up to
+    // 8 rows only in a caller's workspace that holds the fragments: such a
+    // call without one writes nothing into the library's own buffer, so calls
+    // on several streams stay independent.
     const bool skinny_frag = !groups && mode == GEMV_PLAIN && M > 4 && K <= 0x7fffffff &&
                              gemm_skinny_serves((int)M, (int)K, (int)gs, false, false) &&
-                             (!ws || wsb >= layout(M > 8 ? M : 9, Nmax, K, gs).total);
+                             (M > 8 || (ws && wsb >= layout(9, Nmax, K, gs).total));
     if (gemv_path_ok(M, K, gs) && !skinny_frag) {
         // Lane numerics apply per segment shape; segments sharing one launch
         // must agree on the path.

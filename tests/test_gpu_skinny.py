@@ -117,6 +117,31 @@ def test_small_workspace_still_served(orc):
     assert_bits(q.linear_i8(dev(A), dev(W), dev(S), 64, workspace=small), orc.linear(A, W, S, 64), "small workspace")
 
 
+def test_no_workspace_single_launch(orc):
+    """5..8 rows without a workspace keep nothing in the library's own buffer
+    (which two streams would share): one launch, no quantized activations ahead
+    of it. With a workspace the fragments are a launch of their own."""
+    import ctypes
+    M, N, K, gs = 6, 40, 6144, 64
+    A, W, S = make_case(5, M, N, K, gs)
+    a, w, s = dev(A), dev(W), dev(S)
+    ws = torch.zeros(q.workspace_bytes(M, N, K, gs), dtype=torch.uint8, device="cuda")
+    hip = ctypes.CDLL("libamdhip64.so")
+    for workspace, launches in ((None, 1), (ws, 2)):
+        out = q.linear_i8(a, w, s, gs, workspace=workspace)
+        assert_bits(out, orc.linear(A, W, S, gs), "before the capture")
+        g = torch.cuda.CUDAGraph(keep_graph=True)
+        with torch.cuda.graph(g):
+            q.linear_i8(a, w, s, gs, out=out, workspace=workspace)
+        n = ctypes.c_size_t()
+        assert hip.hipGraphGetNodes(ctypes.c_void_p(g.raw_cuda_graph()), None, ctypes.byref(n)) == 0
+        assert n.value == launches
+        out.zero_()
+        g.instantiate()
+        g.replay()
+        assert_bits(out, orc.linear(A, W, S, gs), "replayed")
+
+
 # the wide kernel (csrc/gemm_wide.hip): N * K >= 2^26, each row padding and
 # group size, with fewer tiles than waves and more, ragged rows
 @pytest.mark.parametrize("gs", [32, 64, 128])
