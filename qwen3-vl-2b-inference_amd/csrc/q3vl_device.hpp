@@ -9,6 +9,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <cfloat>
+#include <climits>
 
 #ifndef Q3VL_INLINE
 #define Q3VL_INLINE __device__ __forceinline__
@@ -246,6 +247,23 @@ Q3VL_INLINE int32_t run_sum(int32_t v) {
     if constexpr (WIDTH >= 8) v += dpp_half_mirror(v);
     if constexpr (WIDTH >= 16) v += dpp_mirror(v);
     return v;
+}
+
+// Largest value, smallest integer of the 16 lanes of a DPP row, in each lane.
+Q3VL_INLINE float dpp_f(float v, int32_t (*dpp)(int32_t)) {
+    return __builtin_bit_cast(float, dpp(__builtin_bit_cast(int32_t, v)));
+}
+Q3VL_INLINE float row16_max(float v) {
+    v = fmaxf(v, dpp_f(v, dpp_xor1));
+    v = fmaxf(v, dpp_f(v, dpp_xor2));
+    v = fmaxf(v, dpp_f(v, dpp_half_mirror));
+    return fmaxf(v, dpp_f(v, dpp_mirror));
+}
+Q3VL_INLINE int32_t row16_min(int32_t v) {
+    v = min(v, dpp_xor1(v));
+    v = min(v, dpp_xor2(v));
+    v = min(v, dpp_half_mirror(v));
+    return min(v, dpp_mirror(v));
 }
 
 // One step of scatter_sums over n values: the thread keeps the half of

@@ -86,6 +86,25 @@ def test_argmax_tiles(orc, M, V, gs):
     np.testing.assert_array_equal(ids2.cpu().numpy(), ids.cpu().numpy())
 
 
+@pytest.mark.parametrize("gs", [32, 64, 128])
+@pytest.mark.parametrize("M,V", [(17, 200), (70, 20005)], ids=str)
+def test_argmax_ties_in_a_tile(orc, M, V, gs):
+    """The winning column repeated over the lanes of its own 16-column tile and
+    a row that is all zeros: the lowest column wins; a row of NaN has none."""
+    K = 128
+    A, W, S = make_case(M + V + gs, M, V, K, gs)
+    A[1] = 0.0
+    A[2] = np.nan
+    for r in (0, 5, M - 1):
+        best = int(orc.argmax_rows(orc.linear(A[r:r + 1].repeat(9, 0), W, S, gs))[0])
+        for x in (1, 2, 4, 8, 15):
+            if (best ^ x) < V:
+                W[best ^ x], S[best ^ x] = W[best], S[best]
+    want = orc.linear(A, W, S, gs)
+    ids = q.lm_head_argmax(dev(A), dev(W), dev(S), gs).cpu().numpy()
+    np.testing.assert_array_equal(ids, orc.argmax_rows(want))
+
+
 @pytest.mark.parametrize("M", [1, 4, 40], ids=str)
 def test_silu_range(orc, M):
     """Gates from 2^-75 to past expf's range on both sides, 0, infinite and
