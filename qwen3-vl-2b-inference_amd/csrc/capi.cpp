@@ -210,16 +210,34 @@ int run_linear(const float *A, int nseg, const int8_t *const *W, const float *co
     int rc = resolve_ws(ws, wsb, L.total, &wbase);
     if (rc) return rc;
 
-    // 2..16 rows against a very wide weight (the lm_head over a batch of
-    // rows): MFMA tiles that read the weights once, quantizing inside.
-    bool wide = mode != GEMV_SWIGLU && M <= 16;
-    for (int i = 0; wide && i < nseg; ++i)
-        wide = !(G && G[i]) && (size_t)Ns[i] * K >= ((size_t)1 << 26) &&
-               gemm_wide_serves((int)M, (int)Ns[i], (int)K, (int)gs);
-    if (wide) {
-        int cus = 0;
+    int cus = 0;
+    if (M > 1 || !gemv_path_ok(M, K, gs)) {
         rc = device_cus(&cus);
         if (rc) return rc;
+    }
+    // ---- 2..16 rows. A weight of 2^26 values or more is wide: the lm_head's
+    // kernel takes it where its LDS holds the rows (K up to 6400 at 2..4 rows,
+    // 3328 at 5..8, 2816 at 9..16, a multiple of 256): MFMA tiles that read
+    // the weights once, quantizing inside. Two rows cost the GEMV little more
+    // than one: they stay with it at K = 4096, which fills its block (2 x 16384
+    // 25.9 us against 18.9, 2 x 50000 46.9 against 44.4), at K above 3072 with
+    // fewer than 5 tiles a CU for the kernel's 8 waves (2 x 20000 x 3584 23.9
+    // against 21.1; but 2 x 32768 x 3840 26.8 against 30.0), and at group size
+    // 32 with K of whole waves below 2^28 values (2 x 50000 x 2048 32.2 against
+    // 29.2; but 2 x 151936 x 1280 47.6 against 55.0).
+    bool groups = false, wide_weight = true, wide = mode != GEMV_SWIGLU && M <= 16;
+    size_t tiles = 0, wbytes = 0;
+    for (int i = 0; i < nseg; ++i) {
+        groups = groups || (G && G[i]);
+        tiles += (Ns[i] + 15) / 16;
+        wbytes += Ns[i] * K;
+        wide_weight = wide_weight && Ns[i] * K >= ((size_t)1 << 26);
+        wide = wide && gemm_wide_serves((int)M, (int)Ns[i], (int)K, (int)gs) &&
+               !(M == 2 && ((K > 3072 && K <= 4096 && (K == 4096 || (Ns[i] + 15) / 16 < 5 * (size_t)cus)) ||
+                            (gs == 32 && K % 1024 == 0 && K <= 4096 && Ns[i] * K < (size_t)1 << 28)));
+    }
+    wide = wide && wide_weight && !groups;
+    if (wide) {
         for (int i = 0; i < nseg; ++i) {
             const bool am = mode == GEMV_ARGMAX;
             float *pv = am ? reinterpret_cast<float *>(wbase + L.parts_val) : nullptr;
@@ -233,23 +251,49 @@ int run_linear(const float *A, int nseg, const int8_t *const *W, const float *co
         }
         return Q3VL_OK;
     }
+    // A wide weight past that kernel: the few-row kernel's blocks, one or two
+    // a CU by their LDS, run one after another, and the GEMV is bound by its
+    // dot products; the fragment-order GEMM's blocks take 32 rows in the time.
+    // Measured (us; few-row kernel or its fragment form / GEMV / GEMM): 8 x
+    // 32768 x 4608 64 / 112 / 35, 8 x 50000 x 7168 - / 194 / 88, 16 x 32768 x
+    // 6144 77 / - / 37, 16 x 50000 x 3584 72 / - / 48, 2 x 24000 x 4608 39 / 48 /
+    // 32; but 8 x 50000 x 1024 16 / 29 / 20, 3 x 100000 x 3456 116 / 92 / 103, 16 x
+    // 24000 x 3072 27 / - / 32, 2 x 20000 x 4224 33 / 42 / 38 and at group size 128
+    // 16 x 32768 x 4096 39 / - / 43.
+    // At up to 8 rows where the workspace holds its operand, or where such
+    // calls have always kept it in the library's buffer.
+    const bool swiglu = mode == GEMV_SWIGLU;
+    const bool skinny = !groups && mode != GEMV_ARGMAX &&
+                        gemm_skinny_serves((int)M, (int)K, (int)gs, true, swiglu);
+    const bool one_a_cu = skinny && gemm_skinny_per_cu((int)M, (int)K, (int)gs, true, swiglu) == 1;
+    bool few_gemm = wide_weight && !groups && !swiglu && M <= 16 &&
+                    (M >= 9   ? K > (gs == 128 ? 4096 : 3072)
+                     : M >= 5 ? K > 2048
+                              : one_a_cu && K > 4096 && tiles > 5 * (size_t)cus);
+    if (few_gemm && M <= 8)
+        few_gemm = ws ? wsb >= layout(9, Nmax, K, gs).total
+                      : M >= 5 && (mode == GEMV_ARGMAX || (gs == 64 && K % 512 == 0));
+    for (int i = 0; few_gemm && i < nseg; ++i) few_gemm = gemm_t16_serves((int)M, (int)Ns[i], (int)K, (int)gs);
     // 2..16 rows (plain; 2..8 under SwiGLU): the split-K MFMA kernel, which
     // quantizes the activations itself. Above 8 rows that pays while a CU gets
     // one block of it (9..16 rows x 6144 columns: 11.5 us against 9.3 with a
-    // quantizer launch ahead; x 2048: 6.3 against 7.0).
-    bool groups = false;
-    size_t tiles = 0;
-    for (int i = 0; i < nseg; ++i) {
-        groups = groups || (G && G[i]);
-        tiles += (Ns[i] + 15) / 16;
-    }
-    const bool swiglu = mode == GEMV_SWIGLU;
-    if (!groups && mode != GEMV_ARGMAX && tiles <= 0x7fffffff && K <= 0x7fffffff &&
-        gemm_skinny_serves((int)M, (int)K, (int)gs, true, swiglu)) {
-        int cus = 0;
-        rc = device_cus(&cus);
-        if (rc) return rc;
-        if (M <= 8 || tiles <= (size_t)cus) {
+    // quantizer launch ahead; x 2048: 6.3 against 7.0). Up to K = 4096, where
+    // the GEMV's registers hold a row, 2 to 4 rows are better off on it where
+    // the LDS holds one block a CU and the product takes more than a few
+    // rounds of blocks (few-row kernel / GEMV): 2 x 6144 x 3840 12.9 / 11.7, 2 x
+    // 10000 x 3328 16.3 / 13.2, at group size 128 2 x 8192 x 4096 11.8 / 12.9, 2 x
+    // 10000 x 3328 15.2 / 13.1; 3 x 100000 x 3456 116 / 92, 3 x 20000 x 3456 27.5 /
+    // 26.9; SwiGLU 2 x 8192 x 2048 12.4 / 13.2, 2 x 12288 x 2048 16.7 / 15.5, 2 x
+    // 6144 x 2560 15.0 / 13.1, 3 x 32768 x 2560 54 / 58, 3 x 50000 x 2048 59 / 54,
+    // at group size 128 2 x 8192 x 2944 16.8 / 18.3, 4 x 32768 x 2560 52 / 67.
+    if (skinny && !few_gemm && tiles <= 0x7fffffff) {
+        bool gemv_few = M <= 4 && K <= 4096 && one_a_cu;
+        if (swiglu)
+            gemv_few = gemv_few && (M == 2 ? wbytes > (size_t)cus * ((gs == 128 ? 190 : K > 2048 ? 110 : 140) << 10)
+                                           : gs == 64 && wbytes > (size_t)cus * (768 << 10));
+        else
+            gemv_few = gemv_few && (M == 2 ? tiles > (gs == 64 ? 1 : 2) * (size_t)cus : wbytes > (size_t)cus * (256 << 10));
+        if (!gemv_few && (M <= 8 || tiles <= (size_t)cus)) {
             Q3VL_HIP(launch_gemm_skinny(skinny_args(A, nullptr, nullptr, nseg, W, S, C, Ns, M, K), (int)gs, swiglu, st),
                      "skinny gemm launch");
             return Q3VL_OK;
@@ -259,10 +303,10 @@ int run_linear(const float *A, int nseg, const int8_t *const *W, const float *co
     // 8 rows only in a caller's workspace that holds the fragments: such a
     // call without one writes nothing into the library's own buffer, so calls
     // on several streams stay independent.
-    const bool skinny_frag = !groups && mode == GEMV_PLAIN && M > 4 && K <= 0x7fffffff &&
+    const bool skinny_frag = !groups && !few_gemm && mode == GEMV_PLAIN && M > 4 &&
                              gemm_skinny_serves((int)M, (int)K, (int)gs, false, false) &&
                              (M > 8 || (ws && wsb >= layout(9, Nmax, K, gs).total));
-    if (gemv_path_ok(M, K, gs) && !skinny_frag) {
+    if (gemv_path_ok(M, K, gs) && !skinny_frag && !few_gemm) {
         // Lane numerics apply per segment shape; segments sharing one launch
         // must agree on the path.
         const bool lanes = q3vl_uses_lane_path(M, Ns[0], K);
@@ -321,9 +365,6 @@ int run_linear(const float *A, int nseg, const int8_t *const *W, const float *co
     bool use_t16 = true;
     for (int i = 0; use_t16 && i < nseg; ++i)
         use_t16 = !(G && G[i]) && gemm_t16_serves((int)M, (int)Ns[i], (int)K, (int)gs);
-    int cus = 0;
-    rc = device_cus(&cus);
-    if (rc) return rc;
     if (use_t16 && mode == GEMV_ARGMAX) {
         // a vocabulary of more partials than the workspace holds: refused at
         // group size 64, scanned from stored logits at the others

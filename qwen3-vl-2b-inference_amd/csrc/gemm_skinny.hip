@@ -280,6 +280,10 @@ bool gemm_skinny_serves(int M, int K, int gs, bool fp32, bool swiglu) {
            K <= 1024 * skinny_pieces(skinny_rw(M, fp32), swiglu);
 }
 
+int gemm_skinny_per_cu(int M, int K, int gs, bool fp32, bool swiglu) {
+    return (int)((160 * 1024) / skinny_lds(skinny_rw(M, fp32), K, gs, swiglu));
+}
+
 hipError_t launch_gemm_skinny(const GemmSkinnyArgs &a, int gs, bool swiglu, hipStream_t st) {
     if (!gemm_skinny_serves(a.M, a.K, gs, a.A != nullptr, swiglu) || a.nseg < 1 || a.nseg > 3 || (swiglu && a.nseg != 2) ||
         (!a.A && (!a.Af || !a.asf)))

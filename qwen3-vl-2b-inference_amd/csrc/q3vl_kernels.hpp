@@ -170,6 +170,8 @@ struct GemmSkinnyArgs {
     int nseg, M, K;
 };
 bool gemm_skinny_serves(int M, int K, int gs, bool fp32, bool swiglu);
+// Blocks of it that a CU's LDS holds.
+int gemm_skinny_per_cu(int M, int K, int gs, bool fp32, bool swiglu);
 hipError_t launch_gemm_skinny(const GemmSkinnyArgs &a, int gs, bool swiglu, hipStream_t st);
 
 // 2..16 rows of fp32 activations A [M, K] against a wide weight (K % 256 ==

@@ -159,3 +159,33 @@ def test_wide_few_rows(orc, M, V, K, gs):
     if M <= 8:  # without stored logits
         np.testing.assert_array_equal(q.lm_head_argmax(dev(A), dev(W), dev(S), gs).cpu().numpy(), ids.cpu().numpy())
     assert_bits(q.linear_i8(dev(A), dev(W), dev(S), gs), want, "plain")
+
+
+@pytest.mark.parametrize("gs", [32, 64, 128])
+@pytest.mark.parametrize("M,V,K", [(6, 18749, 3584), (8, 8205, 8192), (3, 20977, 3200), (2, 14567, 4608), (9, 14567, 4608),
+                                   (2, 20977, 3200), (2, 16385, 4096), (2, 20010, 3584)], ids=str)
+def test_wide_past_its_lds(orc, M, V, K, gs):
+    """Wide weights that the wide kernel does not take -- its LDS does not hold
+    the rows, K is no multiple of 256, or 2 rows that are better off on the GEMV
+    -- on whichever kernel they go to, with a workspace and without."""
+    A, W, S = make_case(M + V, M, V, K, gs)
+    W[V - 1], S[V - 1] = W[V // 2], S[V // 2]
+    want = orc.linear(A, W, S, gs)
+    ws = torch.zeros(q.workspace_bytes(M, V, K, gs), dtype=torch.uint8, device="cuda")
+    logits = torch.zeros((M, V), device="cuda")
+    for w in (ws, None):
+        ids = q.lm_head_argmax(dev(A), dev(W), dev(S), gs, logits=logits, workspace=w)
+        assert_bits(logits, want, f"logits {M}x{V}x{K} gs {gs}")
+        np.testing.assert_array_equal(ids.cpu().numpy(), orc.argmax_rows(want))
+        assert_bits(q.linear_i8(dev(A), dev(W), dev(S), gs, workspace=w), want, "plain")
+
+
+@pytest.mark.parametrize("M,N,K", [(3, 51000, 2048), (4, 24001, 3072), (2, 8100, 2048), (2, 9000, 3072)], ids=str)
+def test_swiglu_one_block_a_cu(orc, M, N, K):
+    """SwiGLU where a CU's LDS holds one block of the few-row kernel, on either
+    side of where the GEMV takes over."""
+    A, Wg, Sg = make_case(M + N, M, N, K, 64)
+    _, Wu, Su = make_case(M + N + 1, M, N, K, 64)
+    ws = torch.zeros(q.workspace_bytes(M, N, K, 64), dtype=torch.uint8, device="cuda")
+    got = q.linear_i8_swiglu(dev(A), dev(Wg), dev(Sg), dev(Wu), dev(Su), 64, workspace=ws)
+    assert_bits(got, orc.swiglu(orc.linear(A, Wg, Sg, 64), orc.linear(A, Wu, Su, 64)), f"swiglu {M}x{N}x{K}")
