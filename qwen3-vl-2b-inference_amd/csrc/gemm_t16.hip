@@ -674,10 +674,16 @@ static hipError_t launch_t16(const GemmT16Args &a, hipStream_t st) {
 }
 
 // Which tile. A tile's blocks run in rounds of `cap` blocks a CU; a round of
-// L blocks a CU takes fix + unit[L - 1] * K / 64 us (measured on MI355X at
-// group 64, weights rotating through more than the L2s; group 32 takes 1.15
-// to 1.25 times as long in every tile). The product takes the tile whose
-// rounds cost least. Small products want one small block on every CU, larger
+// L blocks a CU takes fix + unit[L - 1] * K / 64 us, and tail us for each unit
+// of K past the whole loop bodies, which run one at a time (0.3 to 1 us each
+// on top: 65 x 12288 at K = 256 / 384 / 512 takes 10.5 / 13.9 / 12.3 us in
+// tiles of 32 x 128). The plain tables are fitted to the tiles' times, each
+// forced, over 4500 products at groups 32 and 64 and 2200 at 128 (M 17 to
+// 2048, N 512 to 50000, K 128 to 6144, cold caches): the tile taken is 0.3 %
+// (0.5 % at group 128) slower than the best one on average, 22 % at most; with
+// tables read off a few large products, and no tail, it was 1.7 % and 59 %,
+// most of it at K up to 512 (65 x 50000 x 384 32 us, 20.6 in the best tile).
+// The product takes the tile whose rounds cost least. Small products want one small block on every CU, larger
 // ones two or three blocks of 64 x 64, which wait at barriers of their own
 // (4 waves each), and where those leave a round half empty, larger blocks:
 // * plain (us; 32 x 64 / 32 x 128 / 64 x 64 / 64 x 128 / 128 x 128):
@@ -702,39 +708,40 @@ static hipError_t launch_t16(const GemmT16Args &a, hipStream_t st) {
 // two and another launch cost less (at 1501 rows 88 us + 27 in place of 130).
 struct T16Tile {
     int rows, cols, cap;
-    float unit[3], fix;
+    float unit[3], fix, tail;
 };
 struct T16Plan {
     int tile, rows, tile2;  // rows 0 .. rows - 1 by tile, the others (if any) by tile2
 };
 enum { P32x64, P32x128, P64x64, P64x128, P128x128, PLAIN_TILES };
-static const T16Tile kPlain[PLAIN_TILES] = {{32, 64, 1, {0.20f}, 2},
-                                            {32, 128, 1, {0.26f}, 2},
-                                            {64, 64, 3, {0.34f, 0.43f, 0.65f}, 5},
-                                            {64, 128, 2, {0.43f, 0.67f}, 6},
-                                            {128, 128, 1, {0.66f}, 5.5f}};
-static const T16Tile kPlain128[PLAIN_TILES] = {{32, 64, 1, {0.16f}, 2},
-                                               {32, 128, 1, {0.21f}, 2},
-                                               {64, 64, 3, {0.21f, 0.40f, 0.66f}, 5},
-                                               {64, 128, 2, {0.29f, 0.68f}, 6},
-                                               {128, 128, 1, {0.56f}, 5}};
+static const T16Tile kPlain[PLAIN_TILES] = {{32, 64, 1, {0.20f}, 2.5f, 0.3f},
+                                            {32, 128, 1, {0.33f}, 2.5f, 0.55f},
+                                            {64, 64, 3, {0.36f, 0.38f, 0.61f}, 5.2f, 0.7f},
+                                            {64, 128, 2, {0.39f, 0.67f}, 5.3f, 0.48f},
+                                            {128, 128, 1, {0.66f}, 5.7f, 0.97f}};
+static const T16Tile kPlain128[PLAIN_TILES] = {{32, 64, 1, {0.21f}, 3.1f, 0.52f},
+                                               {32, 128, 1, {0.31f}, 2.3f, 0.55f},
+                                               {64, 64, 3, {0.32f, 0.40f, 0.68f}, 9.4f, 0.92f},
+                                               {64, 128, 2, {0.33f, 0.91f}, 5.9f, 0.56f},
+                                               {128, 128, 1, {0.54f}, 4.7f, 0.73f}};
 enum { S32x64L, S32x64, S64x64, S128x128, SWIGLU_TILES };
-static const T16Tile kSwiglu[SWIGLU_TILES] = {{32, 64, 1, {0.18f}, 7},
-                                              {32, 64, 2, {0.20f, 0.36f}, 7},
-                                              {64, 64, 2, {0.35f, 0.61f}, 7.5f},
-                                              {128, 128, 1, {1.16f}, 9}};
+static const T16Tile kSwiglu[SWIGLU_TILES] = {{32, 64, 1, {0.18f}, 7, 0},
+                                              {32, 64, 2, {0.20f, 0.36f}, 7, 0},
+                                              {64, 64, 2, {0.35f, 0.61f}, 7.5f, 0},
+                                              {128, 128, 1, {1.16f}, 9, 0}};
 enum { S32x128, S64x128, SWIGLU128_TILES };
-static const T16Tile kSwiglu128[SWIGLU128_TILES] = {{32, 128, 1, {0.25f}, 8}, {64, 128, 1, {0.55f}, 8}};
+static const T16Tile kSwiglu128[SWIGLU128_TILES] = {{32, 128, 1, {0.25f}, 8, 0}, {64, 128, 1, {0.55f}, 8, 0}};
 
 static T16Plan t16_plan(int M, int N, int K, int gs, bool swiglu, bool argmax, int cus) {
     const T16Tile *tiles = swiglu ? (gs == 128 ? kSwiglu128 : kSwiglu) : gs == 128 ? kPlain128 : kPlain;
     const int n = swiglu ? (gs == 128 ? (int)SWIGLU128_TILES : (int)SWIGLU_TILES) : (int)PLAIN_TILES;
-    const float units = (float)K / 64;
+    const float units = (float)K / 64, tail = (float)(K / (gs == 128 ? 128 : 64) % 4);
     auto cost = [&](const T16Tile &q, int m) {
         const long blocks = (long)((m + q.rows - 1) / q.rows) * ((N + q.cols - 1) / q.cols);
         const long slots = (long)q.cap * cus, rounds = (blocks - 1) / slots;
         const long level = (blocks - rounds * slots - 1) / cus;  // of the last round
-        return (float)rounds * (q.fix + q.unit[q.cap - 1] * units) + q.fix + q.unit[level] * units;
+        return (float)rounds * (q.fix + q.unit[q.cap - 1] * units + q.tail * tail) + q.fix + q.unit[level] * units +
+               q.tail * tail;
     };
     T16Plan best{0, M, 0};
     float least = 1e30f;
@@ -765,6 +772,13 @@ static T16Plan t16_plan(int M, int N, int K, int gs, bool swiglu, bool argmax, i
         }
     }
     return best;
+}
+
+void gemm_t16_tiles(int M, int N, int K, int gs, bool swiglu, bool argmax, int cus, int out[3]) {
+    const T16Plan p = t16_plan(M, N, K, gs, swiglu, argmax, cus);
+    out[0] = p.tile;
+    out[1] = p.rows;
+    out[2] = p.tile2;
 }
 
 // Columns per argmax partial of a plain product.

@@ -147,6 +147,9 @@ hipError_t launch_quantize_t16(const float *A, _Float16 *qf, float *asf, int M, 
 // Whether this GEMM serves an M x N x K product (else launch_gemm's kernel,
 // with launch_quantize_f16).
 bool gemm_t16_serves(int M, int N, int K, int gs);
+// The tile it takes, the rows of it, the tile of the other rows (the tests ask
+// which tiles they reach).
+void gemm_t16_tiles(int M, int N, int K, int gs, bool swiglu, bool argmax, int cus, int out[3]);
 // Columns per argmax partial of a plain product.
 int gemm_t16_argmax_cols(int M, int N, int K, int gs, int cus);
 hipError_t launch_gemm_t16(const GemmT16Args &a, int gs, bool swiglu, int cus, hipStream_t st);

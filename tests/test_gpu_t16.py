@@ -25,10 +25,33 @@ def assert_bits(got, want, what):
     assert bad.size == 0, f"{what}: {bad.size} of {g.size} differ, first at {bad[:5]}"
 
 
-# rows x columns that reach the five plain tiles on 256 CUs (32 x 64, 32 x
-# 128, 64 x 64, 64 x 128, 128 x 128), each with ragged last tiles
+# rows x columns over the plain tiles (32 x 64, 32 x 128, 64 x 64, 64 x 128,
+# 128 x 128), each with ragged last tiles; test_t16_plan.py holds that all of
+# them are reached on 256 CUs
 PLAIN = [(9, 70), (33, 130), (70, 6001), (70, 14003), (70, 20005), (131, 12801), (70, 21851), (131, 16571),
          (131, 19871), (70, 24821)]
+# ... with the K that those need: 128 x 128 in front of a row split at groups 32
+# and 64, 64 x 64 at group 128
+PLAIN_K = [(257, 13311, 64), (140, 22275, 256), (129, 21905, 320), (33, 33824, 1024), (33, 33620, 1152)]
+SWIGLU = [(9, 70), (9, 16571), (40, 16571), (70, 11001), (70, 17003)]
+MLP = [(9, 128, 128), (37, 640, 384), (70, 128, 11008), (70, 128, 17024), (130, 192, 320), (9, 128, 16640),
+       (40, 128, 16640)]
+SPLIT = [(2100, 2048, 512)]
+
+
+def plain_ks(N, gs):
+    """The K of test_linear_tiles: loop bodies' remainders, less than one, one and some."""
+    return [K for K in ((128, 640, 1152) if gs == 128 else (64, 320, 576)) if not (N > 10000 and K > 700)]
+
+
+@pytest.mark.parametrize("gs", [32, 64, 128])
+@pytest.mark.parametrize("M,N,K", PLAIN_K, ids=str)
+def test_linear_tiles_at_k(orc, M, N, K, gs):
+    if K % gs:
+        pytest.skip("not whole groups")
+    A, W, S = make_case(M + N + K, M, N, K, gs)
+    A[0, gs // 2] = 1e30
+    assert_bits(q.linear_i8(dev(A), dev(W), dev(S), gs), orc.linear(A, W, S, gs), f"{M}x{N}x{K} gs {gs}")
 
 
 @pytest.mark.parametrize("gs", [32, 64, 128])
