@@ -128,6 +128,32 @@ def test_argmax_ties_in_a_tile(orc, M, V, gs):
     np.testing.assert_array_equal(ids, orc.argmax_rows(want))
 
 
+# what the fragment-order GEMM leaves to csrc/gemm.hip
+def test_k_past_its_offsets(orc):
+    """K past 2^22 (32-bit offsets into a block's rows): plain and SwiGLU."""
+    M, N, K, gs = 3, 2, (1 << 22) + 64, 64
+    A, Wg, Sg = make_case(1, M, N, K, gs)
+    _, Wu, Su = make_case(2, M, N, K, gs)
+    g, u = orc.linear(A, Wg, Sg, gs), orc.linear(A, Wu, Su, gs)
+    assert_bits(q.linear_i8(dev(A), dev(Wg), dev(Sg), gs), g, "plain")
+    assert_bits(q.linear_i8_swiglu(dev(A), dev(Wg), dev(Sg), dev(Wu), dev(Su), gs), orc.swiglu(g, u), "swiglu")
+
+
+@pytest.mark.parametrize("gs", [32, 64])
+def test_argmax_of_stored_logits(orc, gs):
+    """A vocabulary of more argmax partials than the workspace holds (8192, of
+    128 columns): the logits are stored and scanned."""
+    M, V, K = 9, 8192 * 128 + 65, 64
+    A, W, S = make_case(gs, M, V, K, gs)
+    W[V - 1], S[V - 1] = W[V // 2], S[V // 2]
+    want = orc.linear(A, W, S, gs)
+    ids = q.lm_head_argmax(dev(A), dev(W), dev(S), gs).cpu().numpy()
+    np.testing.assert_array_equal(ids, orc.argmax_rows(want))
+    logits = torch.zeros((M, V), device="cuda")
+    q.lm_head_argmax(dev(A), dev(W), dev(S), gs, logits=logits)
+    assert_bits(logits, want, "logits")
+
+
 @pytest.mark.parametrize("M", [1, 4, 40], ids=str)
 def test_silu_range(orc, M):
     """Gates from 2^-75 to past expf's range on both sides, 0, infinite and
