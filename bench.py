@@ -845,15 +845,16 @@ def pmc_workload():
 
 def pmc_workload_gemm():
     """Workload for the GEMM counter passes: 4 eager calls of each of config
-    2's GEMMs (gate|up with the SwiGLU epilogue, then down, M = 512) and of
-    config 4's vision linears (qkv, proj, fc1, fc2 at M = 784; the merger's
-    fc1 at M = 196), each call its fragment-order quantizer and its
-    gemm_t16_kernel."""
+    2's GEMMs (gate|up with the SwiGLU epilogue, then down, M = 512), the same
+    two at 1501 rows, and config 4's vision linears (qkv, proj, fc1, fc2 at M =
+    784; the merger's two at M = 196), each call its fragment-order quantizer
+    and its gemm_t16_kernel."""
     import torch
     import q3vl_int8 as q
     shapes = [("cfg2 gate|up", 512, 6144, 2048, True), ("cfg2 down", 512, 2048, 6144, False)]
     shapes += [(f"cfg4 {n}", VIS_T, N, K, False) for n, (N, K) in zip(("qkv", "proj", "fc1", "fc2"), VIS_SHAPES)]
-    shapes += [("cfg4 merger fc1", VIS_T // 4, MERGER_SHAPES[0][0], MERGER_SHAPES[0][1], False)]
+    shapes += [(f"cfg4 merger {n}", VIS_T // 4, N, K, False) for n, (N, K) in zip(("fc1", "fc2"), MERGER_SHAPES)]
+    shapes += [("gate|up 1501", 1501, 6144, 2048, True), ("down 1501", 1501, 2048, 6144, False)]
     for name, M, N, K, sw in shapes:
         W, S = gen_weights(N, K, 1, 11)
         A = torch.randn((M, K), dtype=torch.float32, device="cuda")

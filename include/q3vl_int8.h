@@ -32,10 +32,13 @@
  * `stream` (a hipStream_t; NULL = the null stream) and returns a status code;
  * q3vl_last_error() gives the message of this thread's last failure.
  *
- * Shape support: K % group_size == 0. M <= 8 runs the HBM-bound GEMV kernels
- * (group_size in {16,32,64,128,256}, K <= 8192, K % 16 == 0); M > 8 runs the
- * matrix-core GEMM (group_size in {32,64,128}, K % 64 == 0). A and W must be
- * 16-byte aligned.
+ * Shape support: K % group_size == 0. M <= 8: group_size in
+ * {16,32,64,128,256}, K <= 8192, K % 16 == 0 (one row runs an HBM-bound GEMV;
+ * 2..8 rows a few-row matrix-core kernel at group sizes 64 and 128, a wide one
+ * where N * K >= 2^26, or the general GEMM, whichever takes the shape fastest,
+ * and the GEMV elsewhere). M > 8, or M <= 8 past the GEMV's K: the matrix-core
+ * kernels (group_size in {32,64,128}, K % 64 == 0). Which kernel runs changes
+ * no bit of a result. A and W must be 16-byte aligned.
  *
  * Workspace: entry points that need scratch device memory take `workspace`
  * and `workspace_bytes` (>= q3vl_workspace_bytes()). Passing NULL makes the
@@ -43,7 +46,12 @@
  * (not allowed while the stream is being captured into a HIP graph; capture
  * callers pass their own workspace). A caller's workspace must be 256-byte
  * aligned; its contents need no initialization (every call writes what it
- * reads). Calls sharing one workspace must be ordered on one stream.
+ * reads). Calls sharing one workspace must be ordered on one stream, and so
+ * must calls that pass NULL and use the library's buffer: every call of more
+ * than 8 rows or K > 8192, the MLP block, the argmax calls, the decode step,
+ * and products of 5..8 rows with a weight of N * K >= 2^26 at group_size 64.
+ * The other linears of up to 8 rows keep nothing in it, and may run on several
+ * streams without a workspace.
  */
 #ifndef Q3VL_INT8_H
 #define Q3VL_INT8_H
@@ -137,10 +145,11 @@ int q3vl_linear_i8_swiglu(const float *A, const int8_t *Wg, const float *Sg,
  * down linear() call: Y = (silu(A Wg^T) * (A Wu^T)) Wd^T with A [M,H],
  * Wg/Wu [I,H], Wd [H,I], Y [M,H]; the numerics of those four calls (the down
  * projection quantizes h as the reference's linear() quantizes state->gate).
- * With M > 8, group size 64 and H, I multiples of 512, the gate|up GEMM's
- * epilogue quantizes h straight into the down GEMM's operand (no h in
- * memory, one quantizer launch fewer); otherwise the two calls run through
- * an h buffer in the workspace (>= q3vl_mlp_workspace_bytes()). */
+ * With M > 8, group_size in {32,64,128} and H, I multiples of 64 (where the
+ * workspace that q3vl_mlp_workspace_bytes() reports holds both operands), the
+ * gate|up GEMM's epilogue quantizes h straight into the down GEMM's operand
+ * (no h in memory, one quantizer launch fewer); otherwise the two calls run
+ * through an h buffer in the workspace. */
 int q3vl_mlp_i8(const float *A, const int8_t *Wg, const float *Sg,
                 const int8_t *Wu, const float *Su, const int8_t *Wd,
                 const float *Sd, float *Y, size_t M, size_t H, size_t I,

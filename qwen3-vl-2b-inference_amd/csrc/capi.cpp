@@ -75,9 +75,8 @@ WsLayout layout(size_t M, size_t N, size_t K, size_t gs) {
     L.parts_idx = off;
     off += align256(kMaxGemvParts * mm * sizeof(int32_t));
     if (M > 8) {
-        // rows padded to whole 32-row m-tiles (the fragment-order layout of
-        // the group-64 GEMM; the transposed scales of the others use the same
-        // stride)
+        // rows padded to whole 32-row m-tiles (the fragment order; the
+        // transposed scales of gemm.hip use the same stride)
         const size_t Kg = gs ? K / gs : 0;
         const size_t Mpad = (M + 31) & ~(size_t)31;
         L.lda_s = (int)Mpad;
@@ -187,8 +186,10 @@ GemmSkinnyArgs skinny_args(const float *A, const _Float16 *Af, const float *asf,
     return g;
 }
 
-// Shared-activation runner: segments ride one GEMV launch (M <= 8) or one
-// quantization followed by one GEMM per segment (M > 8).
+// Shared-activation runner. One row: the segments ride one GEMV launch. 2..16
+// rows: the wide kernel (a launch a segment), the few-row kernel (one launch,
+// or a quantizer's ahead of it), the GEMV or the general GEMM, as the rules
+// below choose. More rows: one quantization, then one GEMM per segment.
 int run_linear(const float *A, int nseg, const int8_t *const *W, const float *const *S,
                float *const *C, int32_t *const *G, const size_t *Ns, size_t M, size_t K,
                size_t gs, int mode, void *ws, size_t wsb, hipStream_t st, int32_t *ids) {
@@ -345,8 +346,8 @@ int run_linear(const float *A, int nseg, const int8_t *const *W, const float *co
         return fail(Q3VL_ERR_UNSUPPORTED,
                     "GEMM path needs group_size in {32,64,128} and K %% 64 == 0 "
                     "(M=%zu K=%zu group_size=%zu)", M, K, gs);
-    // M > 8 (or an M <= 8 shape the GEMV kernels do not take or that runs
-    // faster on the GEMM): quantize once.
+    // M > 8 (or fewer rows of a shape that the kernels above do not take, or
+    // that is faster here): quantize once.
     const WsLayout LG = layout(M > 8 ? M : 9, Nmax, K, gs);
     if (LG.total > L.total) {
         rc = resolve_ws(ws, wsb, LG.total, &wbase);
@@ -366,8 +367,10 @@ int run_linear(const float *A, int nseg, const int8_t *const *W, const float *co
     for (int i = 0; use_t16 && i < nseg; ++i)
         use_t16 = !(G && G[i]) && gemm_t16_serves((int)M, (int)Ns[i], (int)K, (int)gs);
     if (use_t16 && mode == GEMV_ARGMAX) {
-        // a vocabulary of more partials than the workspace holds: refused at
-        // group size 64, scanned from stored logits at the others
+        // a vocabulary of more partials than the workspace holds is scanned
+        // from stored logits, but at group size 64 with K a multiple of 512 it
+        // is refused, and above 32 rows from half the columns on: what this
+        // entry point has always refused stays refused
         const size_t cols = gs == 64 && K % 512 == 0 && M > 32
                                 ? 64 : (size_t)gemm_t16_argmax_cols((int)M, (int)Ns[0], (int)K, (int)gs, cus);
         const size_t nparts = (Ns[0] + cols - 1) / cols;

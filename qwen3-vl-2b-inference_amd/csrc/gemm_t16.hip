@@ -1,6 +1,6 @@
 // gemm_t16.hip -- int8-weight GEMM for M > 8 at group sizes 32, 64 and 128
-// (gfx950), on 16x16x32 fp16 MFMA tiles with the weights taken straight from
-// their loads into the operands.
+// (gfx950), on 16x16x32 fp16 MFMA tiles; weights and activations reach LDS by
+// loads with an LDS destination, the weights are widened from there.
 //
 // Reference: the general path of linear_int8_fp32s_int32acc_transpose,
 // matmul/src/cpu_f32a_i8f32sb_f32c_avx2.cpp:477-662: for each output and
@@ -14,15 +14,21 @@
 // group whose scale is not finite holds q of 0 and -32768 only: its sums are
 // multiples of 2^15 and exact as well.)
 //
-// What bounds it (probes on MI355X at 2.4 GHz): a SIMD issues one fp32
+// What bounds it. Probes on MI355X at 2.4 GHz: a SIMD issues one fp32
 // instruction of a wave every 4 to 5 cycles with two waves on it (5 to 8 with
 // one), a 16x16x32 MFMA holds the vector pipe for about 9, and a wave's MFMAs
 // and VALU work add up rather than overlap. A 16 x 16 output tile costs per
 // group of 64 two MFMAs, 8 VALU operations of the fold (the reference rounds
 // the product and the sum apart) and its share of widening the weights (16
 // operations a 16-column tile, shared by the block's row tiles): about 25 ns
-// a SIMD, and 29 to 36 measured in the loop. So the kernel is bound by VALU
-// issue, and everything else is kept off the issue slots:
+// a SIMD, and 29 to 36 measured in the loop. Counters: with two waves or more
+// a SIMD and whole rounds of large tiles the two units together are busy three
+// quarters of the time (1280 x 6144 x 2048 SwiGLU: VALU 49 %, MFMA 26 %), at
+// 512 rows about two thirds; with one block a CU a half, and with one wave a
+// SIMD a third (196 x 2048 x 4096: 22 and 9 %), the rest being the group's
+// chain of LDS reads, MFMAs, scaling and folds, which too few waves hide. So
+// the large products come near the issue limit and the small ones wait; for
+// both, everything else is kept off the issue slots:
 // * weights and activations reach LDS by loads with an LDS destination (no
 //   registers, no LDS stores; 170 instead of 224 VGPRs at 128 x 256), waited
 //   for by count;

@@ -146,11 +146,10 @@ def test_gemm_parity(orc, M, N, K, gs):
                                    (1024, 8192, 256), (784, 1024, 1024), (784, 4096, 1024),
                                    (784, 1024, 4096), (196, 4096, 4096)])
 def test_gemm_group64_tiles_parity(orc, M, N, K):
-    """The group-64 MFMA GEMMs: the fragment-order kernel (K a multiple of
-    512) with one m-tile (32 x 128 tiles; 7 rows against the 65600-row
-    weight take the 16-row wide kernel) or several (64 x 64 tiles), a
-    single w_s tile (K = 512) and an odd number of them (K = 1536), and the
-    row-major kernel for the other K; ragged M and N, bit-exact. Every
+    """The MFMA kernels at group size 64: the fragment-order GEMM at one
+    32-row tile and at several (7 rows against the 65600-row weight take the
+    wide kernel, 9 rows the few-row one), K of whole loop bodies (256) and less
+    than one (128); ragged M and N, bit-exact. Every
     vision-encoder linear at its own shape: qkv (784, 3072, 1024), proj
     (784, 1024, 1024), fc1 (784, 4096, 1024), fc2 (784, 1024, 4096), and the
     merger's fc1 (196, 4096, 4096) and fc2 (196, 2048, 4096)."""
@@ -160,9 +159,9 @@ def test_gemm_group64_tiles_parity(orc, M, N, K):
 @pytest.mark.parametrize("M,N,K", [(100, 200, 1024), (333, 1030, 2048), (70, 300, 1536), (1030, 6200, 1024),
                                    (1030, 6200, 128)])
 def test_gemm_swiglu_ragged_parity(orc, M, N, K):
-    """SwiGLU GEMM: 64 x (64 + 64) tiles with 8-group w_s tiles (SG = 8;
-    an odd count, 3, at K = 1536), 128-row tiles once the grid outgrows one
-    round of the device (M = 1030), and the row-major kernel at K = 128."""
+    """SwiGLU on the fragment-order GEMM: the small tiles, the large ones once
+    the grid outgrows a round of the device (M = 1030), K = 128 (less than a
+    loop body); ragged M and N."""
     A, Wg, Sg = make_case(900 + M, M, N, K, 64)
     _, Wu, Su = make_case(901 + M, M, N, K, 64)
     H = host(q.linear_i8_swiglu(dev(A), dev(Wg), dev(Sg), dev(Wu), dev(Su), 64))
@@ -264,11 +263,10 @@ def test_swiglu_fused_parity(orc, M, N, K):
     np.testing.assert_array_equal(H.view(np.uint32), H_ref.view(np.uint32))
 
 
-# The MLP block (q3vl_mlp_i8): fused where M > 8, group 64 and H, I are
-# multiples of 512 (the gate|up GEMM's epilogue quantizes h for the down
-# GEMM, in its 64-row and, at M = 600 x I = 6144, its 128-row tiles; M = 9
-# leaves a block's second m-tile past the product); the two calls through an
-# h buffer elsewhere (M <= 8, I = 1088, group 32).
+# The MLP block (q3vl_mlp_i8): fused where M > 8 and H, I are multiples of 64
+# (the gate|up GEMM's epilogue quantizes h for the down GEMM, in its small and,
+# at M = 600 x I = 6144, its large tiles; M = 9 leaves most of a 32-row tile
+# past the product); the two calls through an h buffer at M <= 8.
 MLP = [(512, 2048, 6144, 64), (100, 1024, 2048, 64), (9, 512, 512, 64), (600, 512, 6144, 64),
        (33, 1024, 1536, 64), (8, 1024, 2048, 64), (64, 1024, 1088, 64), (64, 1024, 1024, 32)]
 
